@@ -9,6 +9,9 @@
 // each 1-DOF joint's axis; it returns the joint accelerations the reference's
 // dynamics_continuous computes with CRBA + RNEA + LU (dynamics.rs:322-364).
 //
+// Serial chains in FP64 run gp_chain_impl.h's dynamics instead (the same
+// algorithm in frames that make each joint's transform two planar rotations).
+//
 // Arithmetic: R = double (FP64 everywhere) or R = float (FP32 kinematics,
 // bias forces, contact forces and both sweeps; the joint-space inertia D,
 // the bias u, the 6x6 floating-base solve and the q/v accumulation in FP64).
@@ -169,19 +172,18 @@ struct Body1 {  // what a 1-DOF body keeps between the sweeps
   int rev;  // 1 revolute, 0 prismatic
 };
 
-// Lane-private LDS tier of the tree parameters that do not stay in
-// registers. Per body (from the first uncached one on): its tree rotation as a
-// unit quaternion and its translation, 7 values, the rotation rebuilt where a
-// sweep uses it (24 operations in place of 9 loads); then, while room is left,
-// the rigid inertias (10 values) of the first of those bodies. One row of
-// `pitch` values per lane (lane-major, so every access is the lane's base
-// register plus an immediate offset; an odd pitch spreads a wave's 64-bit
-// accesses over all banks), written once per launch; a lane reads and writes
-// only its own row, so no barrier is needed. Budget: kLdsLaneBytes per lane,
-// the CU's 160 KB over its 256 lanes at one wave per SIMD (the occupancy of
-// every kernel that has uncached bodies). Without it the FP64 7-joint chain
-// re-reads every body's 22 values in every sweep from beyond L2 (~110 MB per
-// step at 65,536 arms).
+// Lane-private LDS tier of the tree parameters that do not stay in registers
+// (FP32 chains of 10-12 joints; FP64 chains: ChainTier). Per body (from the
+// first uncached one on): its tree rotation as a unit quaternion and its
+// translation, 7 values, the rotation rebuilt where a sweep uses it (24
+// operations in place of 9 loads); then, while room is left, the rigid
+// inertias (10 values) of the first of those bodies. One row of `pitch` values
+// per lane (lane-major, so every access is the lane's base register plus an
+// immediate offset; an odd pitch spreads a wave's accesses over all banks),
+// written once per launch; a lane reads and writes only its own row, so no
+// barrier is needed. Budget: kLdsLaneBytes per lane, the CU's 160 KB over its
+// 256 lanes at one wave per SIMD (the occupancy of every kernel that has
+// uncached bodies).
 constexpr int kLdsLaneBytes = 640;
 template <class Topo, class R, int CN> struct LdsTier {
   static constexpr int lo = CN > Topo::first ? CN : Topo::first;  // first body in the tier
@@ -194,7 +196,6 @@ template <class Topo, class R, int CN> struct LdsTier {
   static constexpr int slots = 7 * NT + 10 * NI;
   static constexpr int pitch = slots > 0 ? (slots | 1) : 0;
   // the inertias of up to 4 more bodies [lo + NI, lo + NI + NR) in registers
-  // (a 7-joint FP64 chain then reads nothing from memory inside a step)
   static constexpr int NR = (NT == U && U - NI <= 4) ? U - NI : 0;
 };
 
@@ -338,30 +339,35 @@ extern __shared__ __align__(16) unsigned char gp_dyn_lds[];
 #endif
 
 // Bodies whose parameters stay in registers for a whole launch without
-// spilling: every body of a chain of up to 9 joints (FP32 sweeps) or 4 (FP64),
-// one fewer with per-lane joint kinds; the first few of a longer chain; a lone
-// free body's one.
+// spilling (FP32 sweeps; FP64 chains: ChainTier): every body of a chain of up
+// to 9 joints, one fewer with per-lane joint kinds; the first few of a longer
+// chain; a lone free body's one.
 #ifndef GP_PCACHE_F32
 #define GP_PCACHE_F32 9
-#endif
-#ifndef GP_PCACHE_F64
-#define GP_PCACHE_F64 4
 #endif
 #ifndef GP_PCACHE_LONG
 #define GP_PCACHE_LONG 6
 #endif
 template <class Topo, class R, bool ALLREV> constexpr int cached_bodies() {
-  constexpr int n_max = (sizeof(R) == 4 ? GP_PCACHE_F32 : GP_PCACHE_F64) - (ALLREV ? 0 : 1);
+  constexpr int n_max = GP_PCACHE_F32 - (ALLREV ? 0 : 1);
   if (Topo::N == 1) return 1;
   if (Topo::dof(Topo::first) != 1) return 0;
   if (Topo::N <= n_max) return Topo::N;
   return sizeof(R) == 4 ? (ALLREV ? GP_PCACHE_LONG : GP_PCACHE_LONG / 2) : 0;
 }
 
+}  // namespace gp
+#include "gp_chain_impl.h"
+namespace gp {
+
+// FP64 chains run gp_chain_impl.h's dynamics
+template <class Topo, class R> constexpr bool chain_kernel() { return IsChain<Topo>::value && sizeof(R) == 8; }
+
 // Bytes of dynamic LDS a launch of `block` lanes needs for the tier of a
 // kernel with this topology and precision.
 template <class Topo, class R, bool ALLREV> constexpr int lds_tier_bytes(int block) {
-  return LdsTier<Topo, R, cached_bodies<Topo, R, ALLREV>()>::pitch * (int)sizeof(R) * block;
+  if constexpr (chain_kernel<Topo, R>()) return ChainTier<Topo, ALLREV>::pitch * (int)sizeof(R) * block;
+  else return LdsTier<Topo, R, cached_bodies<Topo, R, ALLREV>()>::pitch * (int)sizeof(R) * block;
 }
 
 // A lone floating body: its articulated inertia is its rigid inertia, the same
@@ -723,11 +729,112 @@ __device__ __forceinline__ bool fast_step(const BucketArgs& a, const FP& P, int 
   return ok;
 }
 
+// The chain kernels' held torques: in registers for the launch, except where
+// the per-joint state fills the register file (12 joints, or 9-12 with per-lane
+// joint kinds): those read them in each step, from L1.
+template <class Topo, bool ALLREV> constexpr bool chain_tau_reg() {
+  constexpr int J = ChainTier<Topo, ALLREV>::J;
+  return !(J >= 12 || (!ALLREV && J >= 9));
+}
+
+// n_steps semi-implicit Euler (RK = false; integrators.rs:276-319) or RK2 /
+// RK4 steps (RK = true, as fast_rk_body) of an FP64 chain per launch, the state
+// in registers. With `active`, lane l runs min(n_steps, active[l]) steps. A
+// non-finite acceleration leaves v non-finite for good, so one look at q and v
+// after the last step finds it.
+template <class Topo, bool ALLREV, bool RK>
+__device__ __forceinline__ void chain_body(const BucketArgs& a, int inst, double dt, int n_steps, int integrator) {
+  constexpr int J = ChainTier<Topo, ALLREV>::J;
+  if (inst >= a.B) return;
+  const int Bp = a.Bp;
+  int my_steps = n_steps;
+  if (a.active) {  // serving: the slot's remaining horizon
+    const int left = a.active[inst];
+    if (left <= 0) return;
+    my_steps = min(my_steps, left);
+    a.active[inst] = left - my_steps;
+  }
+  const Soa<double> qS(a.q, J, Bp), vS(a.v, J, Bp), tauS(a.tau, J, Bp), vdotS(a.vdot, J, Bp);
+  double q[J], v[J];
+#pragma unroll
+  for (int k = 0; k < J; ++k) q[k] = qS.ld(k, inst);
+#pragma unroll
+  for (int k = 0; k < J; ++k) v[k] = vS.ld(k, inst);
+  const ChainParams<Topo, ALLREV> P(a, inst, (double*)GP_DYN_LDS);
+  constexpr bool TR = chain_tau_reg<Topo, ALLREV>();
+  double tr[TR ? J : 1];
+  if constexpr (TR) {
+#pragma unroll
+    for (int k = 0; k < J; ++k) tr[k] = tauS.ld(k, inst);
+  }
+  auto tau = [&](int k) { return TR ? tr[TR ? k : 0] : tauS.ld(k, inst); };
+  bool ok = true;
+  if constexpr (!RK) {
+    for (int s = 0; s < my_steps; ++s) {
+      const bool last = s + 1 == my_steps;
+      ok = chain_dynamics<Topo, ALLREV>(P, q, v, tau, [&](int j, double qdd) {
+             if (last) vdotS.st(j, inst, qdd);
+             v[j] = v[j] + qdd * dt;
+             q[j] += v[j] * dt;
+           }) && ok;
+    }
+  } else {
+    const bool rk4 = integrator == GP_RUNGE_KUTTA_4;
+    const int stages = rk4 ? 4 : 2;
+    double qs[J], vs[J], ak[J], sum[J];
+    for (int s = 0; s < my_steps; ++s) {
+#pragma unroll
+      for (int k = 0; k < J; ++k) { qs[k] = q[k]; vs[k] = v[k]; }
+#pragma unroll 1
+      for (int st = 0; st < stages; ++st) {
+        ok = chain_dynamics<Topo, ALLREV>(P, qs, vs, tau, [&](int j, double qdd) { ak[j] = qdd; }) && ok;
+        if (st == 0) {
+          if (s + 1 == my_steps) {
+#pragma unroll
+            for (int k = 0; k < J; ++k) vdotS.st(k, inst, ak[k]);
+          }
+#pragma unroll
+          for (int k = 0; k < J; ++k) sum[k] = ak[k];
+        } else if (st < 3) {
+#pragma unroll
+          for (int k = 0; k < J; ++k) sum[k] = sum[k] + ak[k] * 2.0;
+        } else {
+#pragma unroll
+          for (int k = 0; k < J; ++k) sum[k] = (sum[k] + ak[k]) / 6.0;
+        }
+        const double h = st + 1 < stages && st != 2 ? dt / 2.0 : dt;
+        const bool fin = st + 1 == stages;
+#pragma unroll
+        for (int k = 0; k < J; ++k) {
+          const double qn = q[k] + v[k] * h, vn = v[k] + (fin && rk4 ? sum[k] : ak[k]) * h;
+          qs[k] = qn;
+          vs[k] = vn;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < J; ++k) { q[k] = qs[k]; v[k] = vs[k]; }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < J; ++k) {
+    qS.st(k, inst, q[k]);
+    ok = ok && isfinite(q[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < J; ++k) {
+    vS.st(k, inst, v[k]);
+    ok = ok && isfinite(v[k]);
+  }
+  if (!ok) a.fault[inst] = 1;
+}
+
 // n_steps semi-implicit Euler steps per launch with the state in registers;
 // q and v accumulate in FP64. With `active`, lane l runs min(n_steps,
 // active[l]) steps (serving: instances with different horizons).
 template <class Topo, class R, int L, bool CONTACTS, bool ALLREV, bool LDS = false>
 __device__ __forceinline__ void fast_sie_body(const BucketArgs& a, int tid, double dt, int n_steps) {
+  if constexpr (chain_kernel<Topo, R>()) return chain_body<Topo, ALLREV, false>(a, tid, dt, n_steps, 0);
+  else {
   constexpr int NQ = nq_of<Topo>(), NV = nv_of<Topo>();
   const int inst = tid / L;
   const int sub = tid % L;
@@ -751,11 +858,7 @@ __device__ __forceinline__ void fast_sie_body(const BucketArgs& a, int tid, doub
   bool ok = true;
   constexpr int PC = cached_bodies<Topo, R, ALLREV>();
   const FastParams<Topo, R, PC, LDS> P(pick<R>(a.bp, a.bpf), Bp, inst, 0, LDS ? (R*)GP_DYN_LDS : nullptr);
-  // the held torques in registers for the launch, except in the FP64 chains
-  // whose per-body state fills the register file (12 joints, or 9-12 with
-  // per-lane joint kinds): they read them in each step, from L1
-  constexpr bool long64 = sizeof(R) == 8 && (Topo::N >= 12 || (!ALLREV && Topo::N >= 9));
-  constexpr bool tau_reg = (PC == Topo::N || FastParams<Topo, R, PC, LDS>::NT > 0) && !long64;
+  constexpr bool tau_reg = PC == Topo::N || FastParams<Topo, R, PC, LDS>::NT > 0;  // held torques in registers
   LaunchConst<Topo, L, CONTACTS, tau_reg> lc;
   ok = load_launch_const<Topo, R, L, CONTACTS>(a, P, inst, sub, lc);
   for (int s = 0; s < my_steps; ++s)
@@ -773,6 +876,7 @@ __device__ __forceinline__ void fast_sie_body(const BucketArgs& a, int tid, doub
     ok = ok && isfinite(v[k]);
   }
   if (!ok) a.fault[inst] = 1;
+  }
 }
 
 template <class Topo, class R, int L, bool CONTACTS, bool ALLREV>
@@ -803,6 +907,8 @@ __device__ __forceinline__ void euler_stage(const double* q, const double* v, co
 // step's first-stage accelerations, as the plain kernel leaves it.
 template <class Topo, class R, int L, bool CONTACTS, bool ALLREV, bool LDS = false>
 __device__ __forceinline__ void fast_rk_body(const BucketArgs& a, int tid, double dt, int n_steps, int integrator) {
+  if constexpr (chain_kernel<Topo, R>()) return chain_body<Topo, ALLREV, true>(a, tid, dt, n_steps, integrator);
+  else {
   constexpr int NQ = nq_of<Topo>(), NV = nv_of<Topo>();
   const int inst = tid / L;
   const int sub = tid % L;
@@ -868,6 +974,7 @@ __device__ __forceinline__ void fast_rk_body(const BucketArgs& a, int tid, doubl
     ok = ok && isfinite(v[k]);
   }
   if (!ok) a.fault[inst] = 1;
+  }
 }
 
 template <class Topo, class R, int L, bool CONTACTS, bool ALLREV>

@@ -101,6 +101,55 @@ M align_z(const double* a) {
   return cols(b1, b2, a);
 }
 
+// rotation about z by the angle with this cosine and sine
+M rot_z(double c, double s) { return M{{c, -s, 0, s, c, 0, 0, 0, 1}}; }
+
+// Turns every body frame of a chain (its 1-DOF joints are bodies first, first
+// + 1, ..., each the child of the one before) about its own joint axis, z, so
+// that each tree rotation after the first joint's is Rx(alpha) Rz(delta), which
+// the FP64 chain kernels use (gp_chain_impl.h). Writing R = Rz(gamma) Rx(alpha)
+// Rz(beta), body i turns by its child's gamma and delta = beta + that. The
+// joint coordinates do not change. Parallel axes (alpha 0 or pi) take gamma
+// = 0; for nearly parallel ones gamma is badly determined, but the rest is read
+// from R with that gamma taken out, so the product is R to rounding.
+void chain_frames(gp_model& m, int first, std::vector<M>& Al) {
+  auto rot = [&](int i) {
+    M R;
+    std::memcpy(R.a, &m.bp[(size_t)i * NBF + BF_RT], sizeof R.a);
+    return R;
+  };
+  M above = ident();  // the turn of the body before
+  for (int i = first; i < m.n; ++i) {
+    double* P = &m.bp[(size_t)i * NBF];
+    double cf = 1.0, sf = 0.0;  // this body's turn
+    if (i + 1 < m.n) {
+      const M Rc = rot(i + 1);  // column 2: (sin gamma sin alpha, -cos gamma sin alpha, cos alpha)
+      const double h = std::hypot(Rc.a[2], Rc.a[5]);
+      if (h > 0.0) { cf = -Rc.a[5] / h; sf = Rc.a[2] / h; }
+    }
+    const M turn = rot_z(cf, sf);
+    M R = mmul(mT(above), rot(i));
+    if (i > first) {
+      // now R = Rx(alpha) Rz(beta): row 0 (cos beta, -sin beta, 0), column 2 (0, -sin alpha, cos alpha)
+      const double hb = std::hypot(R.a[0], R.a[1]), ha = std::hypot(R.a[5], R.a[8]);
+      const double cb = R.a[0] / hb, sb = -R.a[1] / hb, ca = R.a[8] / ha, sa = -R.a[5] / ha;
+      const double cd = cb * cf - sb * sf, sd = sb * cf + cb * sf;
+      R = M{{cd, -sd, 0, ca * sd, ca * cd, -sa, sa * sd, sa * cd, ca}};
+    } else {
+      R = mmul(R, turn);
+    }
+    std::memcpy(P + BF_RT, R.a, sizeof R.a);
+    mv(mT(above), P + BF_PT, P + BF_PT);
+    const double* j = P + BF_J;
+    const M J = mmul(mmul(mT(turn), M{{j[0], j[3], j[4], j[3], j[1], j[5], j[4], j[5], j[2]}}), turn);
+    P[BF_J + 0] = J.a[0]; P[BF_J + 1] = J.a[4]; P[BF_J + 2] = J.a[8];
+    P[BF_J + 3] = J.a[1]; P[BF_J + 4] = J.a[2]; P[BF_J + 5] = J.a[5];
+    mv(mT(turn), P + BF_C, P + BF_C);
+    Al[i] = mmul(Al[i], turn);
+    above = turn;
+  }
+}
+
 uint64_t fnv(uint64_t h, int64_t x) {
   for (int k = 0; k < 8; ++k) {
     h ^= (uint64_t)((x >> (8 * k)) & 0xff);
@@ -189,6 +238,12 @@ int model_create(const gp_model_desc* d, gp_model** out) {
     P[BF_SK] = jt == GP_JOINT_PRISMATIC ? b.spring_k : 0.0;
     P[BF_SL] = b.spring_l;
   }
+  // the mixed kernels' copy keeps the frames as they are here
+  m->bpf.assign(m->bp.begin(), m->bp.end());
+  // spring contacts hold per-instance state the compiled-topology kernels do not carry
+  m->fast_topo = d->n_spring_contacts > 0 ? -1 : fast_topology_id(n, m->parent.data(), m->dofcls.data(), d->n_contacts);
+  if (m->fast_topo >= 1 && m->fast_topo <= 12) chain_frames(*m, 0, Al);
+  if (m->fast_topo > TOPO_WELDED && m->fast_topo <= TOPO_WELDED + kMaxWeldedJoints) chain_frames(*m, 1, Al);
   // contacts, stably sorted by body (contact.rs:103-128 visits bodies in order)
   std::vector<int> order(d->n_contacts);
   for (int c = 0; c < d->n_contacts; ++c) {
@@ -296,8 +351,6 @@ int model_create(const gp_model_desc* d, gp_model** out) {
   }
   h = fnv(h, m->nh);
   m->sig = h;
-  // spring contacts hold per-instance state the compiled-topology kernels do not carry
-  m->fast_topo = m->nsp > 0 ? -1 : fast_topology_id(n, m->parent.data(), m->dofcls.data(), m->nc);
   *out = m.release();
   return GP_OK;
 }
@@ -379,7 +432,7 @@ int bucket_build(Bucket& b, const std::vector<const gp_model*>& lane_models, boo
       for (int f = 0; f < NBF; ++f) {
         const double x = m->bp[(size_t)i * NBF + f];
         bp[((size_t)f * b.nb + i) * Bp + l] = x;
-        bpf[((size_t)f * b.nb + i) * Bp + l] = (float)x;
+        bpf[((size_t)f * b.nb + i) * Bp + l] = m->bpf[(size_t)i * NBF + f];
       }
     }
     for (int c = 0; c < b.nc; ++c)

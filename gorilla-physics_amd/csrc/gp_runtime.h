@@ -18,7 +18,8 @@ struct gp_model {
   int n = 0, nq = 0, nv = 0, nc = 0, nh = 0;
   double g = 9.81;
   std::vector<int> parent, dofcls, kind, qoff, voff, cstart;
-  std::vector<double> bp;  // [n][NBF]
+  std::vector<double> bp;  // [n][NBF]; a chain's bodies turned about their joint axes (gp_runtime.cpp, chain_frames)
+  std::vector<float> bpf;  // the same in the frames before that turn (the mixed kernels')
   std::vector<double> cp;  // [nc][NCF], sorted by body
   std::vector<double> hp;  // [nh][NHF]
   std::vector<int> contact_order;  // sorted slot -> index in the description

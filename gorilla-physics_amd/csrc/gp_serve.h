@@ -26,6 +26,7 @@ struct PoolPtrs {
 struct ModelDev {
   const int* kind;   // [nb]
   const double* bp;  // [nb][NBF] (aligned-frame body parameters)
+  const float* bpf;  // [nb][NBF] the mixed kernels'
   const double* cp;  // [nc][NCF]
   const double* hp;  // [nh][NHF]
 };

@@ -42,9 +42,8 @@ __global__ void __launch_bounds__(64) admit_kernel(const AdmitTable* __restrict_
     m -= p.nb;
     if (m < nbp) {  // packed [nb][NBF] -> SoA [NBF][nb]
       const int i = m / NBF, f = m % NBF;
-      const double val = md.bp[m];
-      p.bp[((size_t)f * p.nb + i) * Bp + l] = val;
-      p.bpf[((size_t)f * p.nb + i) * Bp + l] = float(val);
+      p.bp[((size_t)f * p.nb + i) * Bp + l] = md.bp[m];
+      p.bpf[((size_t)f * p.nb + i) * Bp + l] = md.bpf[m];
       continue;
     }
     m -= nbp;

@@ -157,20 +157,23 @@ int register_model(gp_server* s, const gp_model* m, int* out) {
   auto it = s->model_index.find(m->serial);
   if (it != s->model_index.end()) { *out = it->second; return GP_OK; }
   const size_t kb = sizeof(int) * (size_t)m->n, bb = sizeof(double) * m->bp.size(),
-               cb = sizeof(double) * m->cp.size(), hb = sizeof(double) * m->hp.size();
-  const size_t o_b = (kb + 255) / 256 * 256, o_c = o_b + (bb + 255) / 256 * 256, o_h = o_c + (cb + 255) / 256 * 256;
+               fb = sizeof(float) * m->bpf.size(), cb = sizeof(double) * m->cp.size(),
+               hb = sizeof(double) * m->hp.size();
+  const size_t o_b = (kb + 255) / 256 * 256, o_f = o_b + (bb + 255) / 256 * 256, o_c = o_f + (fb + 255) / 256 * 256,
+               o_h = o_c + (cb + 255) / 256 * 256;
   char* d = nullptr;
   int st = arena_alloc(s, o_h + hb + 8, &d);
   if (st) return st;
   std::vector<char> h(o_h + hb + 8, 0);
   std::memcpy(h.data(), m->kind.data(), kb);
   if (bb) std::memcpy(h.data() + o_b, m->bp.data(), bb);
+  if (fb) std::memcpy(h.data() + o_f, m->bpf.data(), fb);
   if (cb) std::memcpy(h.data() + o_c, m->cp.data(), cb);
   if (hb) std::memcpy(h.data() + o_h, m->hp.data(), hb);
   hipError_t e = hipMemcpy(d, h.data(), h.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) return fail(GP_ERR_DEVICE, "model upload: %s", hipGetErrorString(e));
-  s->models.push_back(ModelDev{(const int*)d, (const double*)(d + o_b), (const double*)(d + o_c),
-                               (const double*)(d + o_h)});
+  s->models.push_back(ModelDev{(const int*)d, (const double*)(d + o_b), (const float*)(d + o_f),
+                               (const double*)(d + o_c), (const double*)(d + o_h)});
   const int idx = (int)s->models.size() - 1;
   s->model_index.emplace(m->serial, idx);
   s->models_dirty = true;

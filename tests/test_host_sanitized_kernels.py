@@ -299,3 +299,58 @@ def test_compiled_kernels_in_bounds_and_match_the_oracle(gp, oracle, host_binary
         assert max(eq.max(), ev.max(), ea.max()) <= 1e-10
     else:
         assert eq.max() <= 1e-5 and ev.max() <= 2e-3 and ea.max() <= 2e-3
+
+
+def _turned_chain(gp, rng, joints, turn, welded, prismatic):
+    """A chain (behind a welded base if asked) whose tree rotations are random
+    ("any"), about the joint axis ("parallel"), half a turn about x
+    ("opposed"), or a hair off parallel (a tilt in radians); axes random unit
+    vectors for "any", +-z otherwise."""
+    from gorilla_physics_amd import abi
+    from gorilla_physics_amd.mechanism import (Isometry3, JointSpring, ModelDesc, SpatialInertia, UnitQuaternion,
+                                               body_desc)
+
+    def rotation():
+        if turn == "any":
+            x = rng.normal(size=3)
+            return UnitQuaternion.from_axis_angle(x / np.linalg.norm(x), rng.uniform(-np.pi, np.pi))
+        about_z = UnitQuaternion.from_axis_angle([0.0, 0.0, 1.0], rng.uniform(-np.pi, np.pi))
+        tilt = 0.0 if turn == "parallel" else np.pi if turn == "opposed" else float(turn)
+        return UnitQuaternion.from_axis_angle([1.0, 0.0, 0.0], tilt) * about_z
+
+    bodies = []
+    for i in range(joints + welded):
+        inertia = SpatialInertia.cuboid_at(rng.uniform(-0.1, 0.1, 3), rng.uniform(0.5, 2.0), *rng.uniform(0.1, 0.4, 3),
+                                           f"b{i}")
+        axis = rng.normal(size=3) if turn == "any" else np.array([0.0, 0.0, rng.choice([-1.0, 1.0])])
+        kind = abi.GP_JOINT_FIXED if welded and i == 0 else abi.GP_JOINT_REVOLUTE
+        spring = None
+        if prismatic and kind == abi.GP_JOINT_REVOLUTE and rng.random() < 0.4:
+            kind, spring = abi.GP_JOINT_PRISMATIC, JointSpring(rng.uniform(5.0, 50.0), 0.1)
+        bodies.append(body_desc(i - 1, kind, axis / np.linalg.norm(axis), Isometry3(rotation(), rng.uniform(-0.3, 0.3, 3)),
+                                inertia, spring))
+    return ModelDesc(bodies, [], [])
+
+
+@pytest.mark.parametrize("turn", ["any", "parallel", "opposed", "1e-8", "1e-16"])
+def test_chain_frames_match_the_oracle(gp, oracle, host_binary_fast, tmp_path, turn):
+    """Chains of 1-12 joints and welded arms of 1-7 whose tree rotations are
+    general, exactly parallel, opposed or nearly parallel (the turn of the
+    bodies' frames about their axes is then undetermined or badly determined),
+    revolute and with sprung prismatic joints: one FP64 step (SIE and RK4)
+    within the 1e-10 per-step bound of the oracle."""
+    from gpu_helpers import step_errors
+    rng = np.random.default_rng(11)
+    descs = [_turned_chain(gp, rng, j, turn, w, p) for p in (False, True)
+             for w, top in ((0, 12), (1, 7)) for j in range(1, top + 1)]
+    q = rng.uniform(-1.5, 1.5, sum(d.nq for d in descs))
+    v = rng.normal(0.0, 0.5, sum(d.nv for d in descs))
+    tau = rng.normal(0.0, 0.2, v.size)
+    for integrator in (0, 2):
+        out = tmp_path / f"out{integrator}.bin"
+        _run(host_binary_fast, tmp_path, out=out, kernel=2, precision=0, models=descs, counts=[1] * len(descs), q=q,
+             v=v, tau=tau, dt=1e-3, integrator=integrator, steps=1, spl=1)
+        q1, v1, a1, _ = _read_out(out, q.size, v.size)
+        eq, ev, ea = step_errors(oracle, descs, q, v, tau, q1, v1, a1, 1e-3, integrator)
+        print(f"turned chains {turn}, integrator {integrator}: {eq.max():.3g} {ev.max():.3g} {ea.max():.3g}")
+        assert max(eq.max(), ev.max(), ea.max()) <= 1e-10
