@@ -198,9 +198,18 @@ constexpr int kVsBodyMaxCandidates = 8;
 constexpr int kVsBodyBlock = 64;
 int launch_vs_body(const BucketArgs& a, double dt, int ccd, int n_steps, int lanes, int candidates, int block,
                    void* stream);
-// rows x B values between a bucket's SoA rows and a flat instance-major array
-// (lane l's values start at flat + flat_off[l]); to_soa = 1: flat -> SoA.
-int launch_flat_xfer(double* soa, int Bp, int B, int rows, const int64_t* flat_off, double* flat, int to_soa,
+// One array of one bucket in a transfer launch: its rows x B values and where
+// each lane's begin in the flat instance-major array (the call's first or
+// second one); first: the entry's first workgroup (64 lanes each).
+struct XferEntry {
+  double* soa;
+  const int64_t* off;
+  int Bp, B, rows;
+  int second;
+  unsigned first;
+};
+// Every entry of a table in one launch; to_soa = 1: flat -> SoA.
+int launch_flat_xfer(const XferEntry* d_table, int n, unsigned blocks, double* flat0, double* flat1, int to_soa,
                      void* stream);
 
 }  // namespace gp

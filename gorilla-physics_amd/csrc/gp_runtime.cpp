@@ -846,6 +846,26 @@ int gp_batch_create(gp_model* const* models, const int64_t* counts, int32_t n_mo
       HIP_TRY(hipMalloc((void**)&b.d_flat_off, off.size() * sizeof(int64_t)));
       HIP_TRY(hipMemcpy(b.d_flat_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     }
+    // and the tables of those calls (state, torques, accelerations)
+    std::vector<XferEntry> xt;
+    for (int which = 0; which < 3; ++which) {
+      gp_batch::Xfer& x = bt->xfer[which];
+      x.at = (int)xt.size();
+      auto add = [&](const Bucket& b, double* soa, int rows, bool second) {
+        if (rows == 0) return;
+        xt.push_back(XferEntry{soa, b.d_flat_off + (second ? b.B : 0), b.Bp, b.B, rows, second ? 1 : 0, x.blocks});
+        x.blocks += (unsigned)((b.B + 63) / 64);
+      };
+      for (const Bucket& b : bt->buckets) {
+        if (which == 0) add(b, b.d_q, b.nq, false);
+        add(b, which == 0 ? b.d_v : which == 1 ? b.d_tau : b.d_vdot, b.nv, true);
+      }
+      x.n = (int)xt.size() - x.at;
+    }
+    if (!xt.empty()) {
+      HIP_TRY(hipMalloc((void**)&bt->d_xfer, xt.size() * sizeof(XferEntry)));
+      HIP_TRY(hipMemcpy(bt->d_xfer, xt.data(), xt.size() * sizeof(XferEntry), hipMemcpyHostToDevice));
+    }
     HIP_TRY(hipStreamCreate(&bt->stream));
     HIP_TRY(hipEventCreate(&bt->ev0));
     HIP_TRY(hipEventCreate(&bt->ev1));
@@ -946,15 +966,10 @@ static int transfer_dev(gp_batch* bt, const double* q, const double* v, double* 
   hipStream_t s = stream ? (hipStream_t)stream : bt->stream;
   if (stream) bt->foreign_stream = true;
   const bool to_dev = oq == nullptr && ov == nullptr;
-  for (Bucket& b : bt->buckets) {
-    int e = 0;
-    if (which == 0)
-      e = launch_flat_xfer(b.d_q, b.Bp, b.B, b.nq, b.d_flat_off, to_dev ? const_cast<double*>(q) : oq, to_dev, s);
-    if (e) return fail(GP_ERR_DEVICE, "transposition launch: %s", hipGetErrorString((hipError_t)e));
-    double* dv = which == 0 ? b.d_v : which == 1 ? b.d_tau : b.d_vdot;
-    e = launch_flat_xfer(dv, b.Bp, b.B, b.nv, b.d_flat_off + b.B, to_dev ? const_cast<double*>(v) : ov, to_dev, s);
-    if (e) return fail(GP_ERR_DEVICE, "transposition launch: %s", hipGetErrorString((hipError_t)e));
-  }
+  const gp_batch::Xfer& x = bt->xfer[which];
+  const int e = launch_flat_xfer(bt->d_xfer + x.at, x.n, x.blocks, to_dev ? const_cast<double*>(q) : oq,
+                                 to_dev ? const_cast<double*>(v) : ov, to_dev, s);
+  if (e) return fail(GP_ERR_DEVICE, "transposition launch: %s", hipGetErrorString((hipError_t)e));
   return GP_OK;
 }
 

@@ -132,4 +132,12 @@ struct gp_batch {
   gp::GroupTable* d_group = nullptr;
   int group_blocks = 0, group_block = 0;
   bool group_valid = false;
+  // device tables of the transfers between flat device arrays and the buckets:
+  // state (q and v), torques, accelerations, each one launch
+  struct Xfer { int at = 0, n = 0; unsigned blocks = 0; };
+  gp::XferEntry* d_xfer = nullptr;
+  Xfer xfer[3];
+  ~gp_batch() {
+    if (d_xfer) (void)hipFree(d_xfer);
+  }
 };
