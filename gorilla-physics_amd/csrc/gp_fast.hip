@@ -27,14 +27,15 @@ int fast_topology_id(int nb, const int* parent, const int* dofcls, int nc) {
   bool quad = nb == 13 && nc == 0;
   for (int i = 0; i < nb && quad; ++i) quad = parent[i] == TopoQuad::parent(i) && dofcls[i] == TopoQuad::dof(i);
   if (quad) return TOPO_QUAD;
-  if (tree_topology_ok(nb, parent)) return TOPO_TREE;
+  if (nb >= 13 && tree_topology_ok(nb, parent)) return TOPO_TREE;
   return -1;
 }
 
 int launch_fast_step(int topo_id, int precision, const BucketArgs& a, double dt, int n_steps, int block,
                      void* stream) {
   if (a.B == 0 || n_steps <= 0) return 0;
-  if (block <= 0) block = 256;
+  // trees: one wave per workgroup, so that their LDS fills a compute unit evenly
+  if (block <= 0) block = topo_id == TOPO_TREE ? 64 : 256;
   hipStream_t s = (hipStream_t)stream;
   if (precision == GP_PREC_MIXED) return launch_fast_f32(topo_id, a, dt, n_steps, block, s);
   return launch_fast_f64(topo_id, a, dt, n_steps, block, s);

@@ -1242,12 +1242,7 @@ __device__ __forceinline__ void grouped_dispatch(const BucketArgs& a, int topo, 
       }
       break;
     case TOPO_TREE:
-      switch (a.lanes) {
-        case 16: wave_tree_body<R, 16>(a, tid, dt, n); break;
-        case 32: wave_tree_body<R, 32>(a, tid, dt, n); break;
-        case 64: wave_tree_body<R, 64>(a, tid, dt, n); break;
-        default: break;
-      }
+      wave_tree_body<R>(a, tid, dt, n);
       break;
     case TOPO_FREE:
       switch (a.lanes) {
@@ -1285,8 +1280,8 @@ template <class R> constexpr int grouped_tier_lane_bytes() {
   constexpr int a = max_tier_lane_bytes<R, true>(std::make_integer_sequence<int, 12>{});
   constexpr int b = max_tier_lane_bytes<R, false>(std::make_integer_sequence<int, 12>{});
   constexpr int m = a > b ? a : b;
-  // the tree kernel's exchange slots share the same LDS in a grouped launch
-  static_assert(m >= kTreeSlotBytes, "grouped LDS row smaller than a tree exchange slot");
+  // the tree kernel's slots share the same LDS in a grouped launch
+  static_assert(m >= kTreeLaneBytes, "grouped LDS row smaller than a tree lane's share");
   return m;
 }
 

@@ -107,6 +107,10 @@ struct BucketArgs {
   const int* qoff;    // [nb]
   const int* voff;    // [nb]
   const int* cstart;  // [nb + 1] contacts sorted by body
+  const int* depth;   // [nb] bodies between this one and its root
+  const int* child_start;  // [nb + 1] children of each body, in index order
+  const int* child;        // [nb]
+  int max_depth;
   // parameters
   const int* kind;     // [nb][Bp]
   const double* bp;    // [NBF][nb][Bp]
@@ -146,7 +150,8 @@ struct GroupTable {
 };
 
 // Compile-time topologies besides the chains (whose id is their body count);
-// TOPO_TREE: any tree of 13 to 64 bodies, one body per lane (gp_tree_impl.h);
+// TOPO_TREE: any other tree of 13 to 64 bodies, one body per lane
+// (gp_tree_impl.h; smaller ones run the same kernel, see bucket_aux_tree);
 // TOPO_WELDED + k: a body welded to the world and a chain of k one-DOF joints
 // behind it, k = 1..7 (a fixed-base manipulator).
 enum { TOPO_FREE = 100, TOPO_QUAD = 101, TOPO_TREE = 102, TOPO_WELDED = 200 };
@@ -155,18 +160,29 @@ constexpr int kMaxWeldedJoints = 7;
 // Lanes per instance of a FAST bucket: free bodies with contacts split their
 // contact points over lanes_per_mech lanes (0 = 4); the quadruped tree runs one
 // lane per leg unless lanes_per_tree is 1.
-// A TOPO_TREE bucket runs one body per lane on 16, 32 or 64 lanes per
-// instance (the power of two that holds its bodies).
+// A TOPO_TREE bucket runs one body per lane.
 inline int fast_lanes(int fast_topo, int lanes_per_mech, int lanes_per_tree, int nb = 0) {
   if (fast_topo == TOPO_FREE) return lanes_per_mech > 0 ? lanes_per_mech : 4;
   if (fast_topo == TOPO_QUAD) return lanes_per_tree == 1 ? 1 : 4;
-  if (fast_topo == TOPO_TREE) return nb <= 16 ? 16 : nb <= 32 ? 32 : 64;
+  if (fast_topo == TOPO_TREE) return nb;
   return 1;
+}
+// Threads that B instances of `lanes` lanes take: trees fill a wave with whole
+// instances and leave its last lanes idle.
+inline int64_t fast_threads(int fast_topo, int64_t B, int lanes) {
+  if (fast_topo != TOPO_TREE) return B * lanes;
+  const int ipw = 64 / lanes;
+  return (B + ipw - 1) / ipw * 64;
 }
 
 // Host-side launchers (gp_plain.hip, gp_fast.hip). Each returns a hipError_t as int.
 int launch_grouped_step(const GroupTable* d_table, int n_blocks, int precision, double dt, int n_steps, int block,
                         void* stream);
+// The same for a table of tree buckets only.
+int launch_grouped_trees(const GroupTable* d_table, int n_blocks, int lds_per_wave, int precision, double dt,
+                         int n_steps, int block, void* stream);
+bool aux_tree_ok(int nb, const int* parent);          // whether the tree kernel takes this topology
+int tree_lds_per_wave(int nb, int floating);          // LDS bytes of its wave
 int launch_plain_step(const BucketArgs& a, double dt, int integrator, int dynamics_only, int n_steps, void* stream);
 // Fast kernels: topo_id from fast_topology_id(); precision GP_PREC_*.
 int fast_topology_id(int nb, const int* parent, const int* dofcls, int nc);

@@ -9,6 +9,7 @@
 // forces follow contact.rs:97-129,260-338 with the half-space test of
 // halfspace.rs:39-44. Per-body intermediates live in device scratch as
 // structure-of-arrays ([field][body][lane]), so every access is coalesced.
+#include "gp_fast_impl.h"
 #include "gp_plain_impl.h"
 
 namespace gp {
@@ -65,6 +66,22 @@ __global__ void __launch_bounds__(256) plain_step_kernel(BucketArgs a, double dt
     if (!ok) a.fault[lane] = 1;
   }
 }
+
+// Buckets of trees (runtime topology, one body per lane: gp_tree_impl.h)
+int launch_grouped_trees(const GroupTable* d_table, int n_blocks, int lds_per_wave, int precision, double dt,
+                         int n_steps, int block, void* stream) {
+  if (n_blocks <= 0 || n_steps <= 0) return 0;
+  const dim3 grid(n_blocks), blk(block);
+  const unsigned lds = (unsigned)(block / 64 * lds_per_wave);
+  if (precision == GP_PREC_MIXED)
+    hipLaunchKernelGGL(grouped_tree_kernel<float>, grid, blk, lds, (hipStream_t)stream, d_table, dt, n_steps);
+  else
+    hipLaunchKernelGGL(grouped_tree_kernel<double>, grid, blk, lds, (hipStream_t)stream, d_table, dt, n_steps);
+  return (int)hipGetLastError();
+}
+
+bool aux_tree_ok(int nb, const int* parent) { return tree_topology_ok(nb, parent); }
+int tree_lds_per_wave(int nb, int floating) { return tree_wave_bytes(nb, floating); }
 
 size_t plain_scratch_doubles(int nb, int nq, int nv, int Bp) {
   return ((size_t)NPF * nb + nq + 5 * (size_t)nv) * Bp;

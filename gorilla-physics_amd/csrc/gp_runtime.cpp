@@ -365,6 +365,7 @@ void Bucket::release() {
   d_arena = nullptr;
   d_flat_off = nullptr;
   d_sstart = nullptr;
+  d_depth = d_child_start = d_child = nullptr;
   d_sp = d_ss = nullptr;
   d_sphere_of = nullptr;
   d_shp = nullptr;
@@ -404,7 +405,8 @@ int bucket_build(Bucket& b, const std::vector<const gp_model*>& lane_models, boo
                o_v = take(8 * nv1 * Bp), o_tau = take(8 * nv1 * Bp), o_tau_tmp = take(8 * nv1 * Bp),
                o_vdot = take(8 * nv1 * Bp), o_fault = take(4 * Bp), o_sstart = take(4 * (b.nb + 1)),
                o_sp = take(8 * NSF * b.nsp * Bp), o_ss = take(8 * NSS * b.nsp * Bp),
-               o_sphere_of = take(4 * b.nb), o_shp = take(8 * NSH * b.ns * Bp), o_rounds = take(4 * Bp);
+               o_sphere_of = take(4 * b.nb), o_shp = take(8 * NSH * b.ns * Bp), o_rounds = take(4 * Bp),
+               o_depth = take(4 * b.nb), o_child_start = take(4 * (b.nb + 1)), o_child = take(4 * b.nb);
   std::vector<char> h(at, 0);
   auto put = [&](size_t off, const void* src, size_t bytes) { if (bytes) std::memcpy(h.data() + off, src, bytes); };
   put(o_parent, b.parent.data(), 4 * b.nb);
@@ -413,6 +415,18 @@ int bucket_build(Bucket& b, const std::vector<const gp_model*>& lane_models, boo
   put(o_cstart, b.cstart.data(), 4 * (b.nb + 1));
   put(o_sstart, b.sstart.data(), 4 * (b.nb + 1));
   put(o_sphere_of, b.sphere_of.data(), 4 * b.nb);
+  // depths and children of the bodies, for the tree kernel
+  int* depth = (int*)(h.data() + o_depth);
+  int* child_start = (int*)(h.data() + o_child_start);
+  int* child = (int*)(h.data() + o_child);
+  b.max_depth = 0;
+  for (int i = 0, at_child = 0; i < b.nb; ++i) {
+    depth[i] = b.parent[i] < 0 ? 0 : depth[b.parent[i]] + 1;
+    b.max_depth = std::max(b.max_depth, depth[i]);
+    for (int k = i + 1; k < b.nb; ++k)
+      if (b.parent[k] == i) child[at_child++] = k;
+    child_start[i + 1] = at_child;
+  }
   double* shp = (double*)(h.data() + o_shp);
   double* sp = (double*)(h.data() + o_sp);
   int* kind = (int*)(h.data() + o_kind);
@@ -470,6 +484,7 @@ int bucket_build(Bucket& b, const std::vector<const gp_model*>& lane_models, boo
   b.d_tau_tmp = (double*)(d + o_tau_tmp); b.d_vdot = (double*)(d + o_vdot); b.d_fault = (int*)(d + o_fault);
   b.d_sstart = (int*)(d + o_sstart); b.d_sp = (double*)(d + o_sp); b.d_ss = (double*)(d + o_ss);
   b.d_sphere_of = (int*)(d + o_sphere_of); b.d_shp = (double*)(d + o_shp); b.d_rounds = (int*)(d + o_rounds);
+  b.d_depth = (int*)(d + o_depth); b.d_child_start = (int*)(d + o_child_start); b.d_child = (int*)(d + o_child);
   b.arena_bytes = at;
   return GP_OK;
 }
@@ -513,6 +528,7 @@ BucketArgs bucket_args(const Bucket& b, int lanes, const double* tau) {
   a.active = b.d_active; a.scratch = b.d_scratch;
   a.nsp = b.nsp; a.sstart = b.d_sstart; a.sp = b.d_sp; a.ss = b.d_ss;
   a.ns = b.ns; a.sphere_of = b.d_sphere_of; a.shp = b.d_shp; a.no_springs = 0;
+  a.depth = b.d_depth; a.child_start = b.d_child_start; a.child = b.d_child; a.max_depth = b.max_depth;
   return a;
 }
 
@@ -554,14 +570,41 @@ static int bucket_lanes(const gp_batch_opts& o, const Bucket& b, int integrator)
   const int tree = integrator == GP_SEMI_IMPLICIT_EULER ? o.lanes_per_tree : 1;
   return fast_lanes(b.fast_topo, o.lanes_per_mech, tree, b.nb);
 }
-static int group_block_size(const gp_batch_opts& o) { return o.block_size > 0 ? o.block_size : 128; }
+// Whether a bucket that has no compiled topology runs the tree kernel instead
+// of the plain one: any tree that it can take, by the automatic choice of
+// kernel, semi-implicit Euler, without spring contacts (per-instance contact
+// state that it does not carry). It was faster at every size tried: twenty
+// steps of 12-body trees, plain against tree kernel, 1 instance 1,893 / 222 us,
+// 65,536 instances 6,398 / 2,743 us; of 2-body ones 342 / 97 and 676 / 193.
+// FP64 whatever the precision option, as the plain kernel.
+static bool bucket_aux_tree(const gp_batch_opts& o, const Bucket& b, int integrator) {
+  return o.kernel == GP_KERNEL_AUTO && b.fast_topo < 0 && integrator == GP_SEMI_IMPLICIT_EULER && b.nsp == 0 &&
+         aux_tree_ok(b.nb, b.parent.data());
+}
 
-// Number of FAST buckets that one grouped launch would cover (0 = no grouping).
+// The grouped launch covers the FAST buckets. If all of them are trees, it is
+// the tree kernel's own (two waves per SIMD instead of the general one's one)
+// and takes the FP64 buckets of bucket_aux_tree too.
+static bool group_is_trees(const gp_batch* bt, int integrator) {
+  for (const Bucket& b : bt->buckets)
+    if (bucket_is_fast(bt->opts, b, integrator) && b.fast_topo != TOPO_TREE) return false;
+  return true;
+}
+static bool in_group(const gp_batch_opts& o, const Bucket& b, int integrator, bool trees) {
+  return bucket_is_fast(o, b, integrator) ||
+         (trees && o.precision == GP_PREC_F64 && bucket_aux_tree(o, b, integrator));
+}
+static int group_block_size(const gp_batch_opts& o, bool trees) {
+  return o.block_size > 0 ? o.block_size : trees ? 64 : 128;
+}
+
+// Number of buckets that one grouped launch would cover (0 = no grouping).
 static int grouped_count(const gp_batch* bt, int integrator) {
   const gp_batch_opts& o = bt->opts;
   if (o.separate_launches || integrator != GP_SEMI_IMPLICIT_EULER) return 0;
+  const bool trees = group_is_trees(bt, integrator);
   int n = 0;
-  for (const Bucket& b : bt->buckets) n += bucket_is_fast(o, b, integrator) ? 1 : 0;
+  for (const Bucket& b : bt->buckets) n += in_group(o, b, integrator, trees) ? 1 : 0;
   return (n >= 2 && n <= kMaxGroup) ? n : 0;
 }
 
@@ -569,7 +612,8 @@ static int grouped_count(const gp_batch* bt, int integrator) {
 // must run before any graph capture.
 static int ensure_group(gp_batch* bt, int integrator) {
   const gp_batch_opts& o = bt->opts;
-  const int block = group_block_size(o);
+  const bool trees = group_is_trees(bt, integrator);
+  const int block = group_block_size(o, trees);
   if (bt->group_valid && bt->group_block == block) return GP_OK;
   GroupTable t{};
   int blocks = 0;
@@ -577,18 +621,23 @@ static int ensure_group(gp_batch* bt, int integrator) {
   // ones do not form the launch's tail
   std::vector<const Bucket*> order;
   for (const Bucket& b : bt->buckets)
-    if (bucket_is_fast(o, b, integrator)) order.push_back(&b);
+    if (in_group(o, b, integrator, trees)) order.push_back(&b);
   const int tree = integrator == GP_SEMI_IMPLICIT_EULER ? o.lanes_per_tree : 1;
   std::stable_sort(order.begin(), order.end(), [&](const Bucket* x, const Bucket* y) {
+    // a tree's step time follows its depth
+    if (trees) return x->max_depth > y->max_depth;
     return bucket_step_cost(*x, o.precision, tree) > bucket_step_cost(*y, o.precision, tree);
   });
+  bt->group_lds = 0;
   for (const Bucket* bb : order) {
     const Bucket& b = *bb;
-    const int lanes = bucket_lanes(o, b, integrator);
+    const int topo = trees ? (int)TOPO_TREE : b.fast_topo;
+    const int lanes = trees ? b.nb : bucket_lanes(o, b, integrator);
     t.args[t.n] = bucket_args(b, lanes, nullptr);
-    t.topo[t.n] = b.fast_topo;
+    t.topo[t.n] = topo;
     t.block_start[t.n] = blocks;
-    blocks += (int)(((int64_t)b.B * lanes + block - 1) / block);
+    blocks += (int)((fast_threads(topo, b.B, lanes) + block - 1) / block);
+    if (trees) bt->group_lds = std::max(bt->group_lds, tree_lds_per_wave(b.nb, b.nq - b.nv));
     ++t.n;
   }
   t.block_start[t.n] = blocks;
@@ -599,6 +648,7 @@ static int ensure_group(gp_batch* bt, int integrator) {
   HIP_TRY(hipMemcpy(bt->d_group, &t, sizeof t, hipMemcpyHostToDevice));
   bt->group_blocks = blocks;
   bt->group_block = block;
+  bt->group_trees = trees;
   bt->group_valid = true;
   return GP_OK;
 }
@@ -627,7 +677,9 @@ static int batch_launch_all(gp_batch* bt, double dt, int integrator, int n_steps
     int spl = o.steps_per_launch > 0 ? o.steps_per_launch : 100;
     for (int done = 0; done < n_steps; done += spl) {
       int n = std::min(spl, n_steps - done);
-      int e = launch_grouped_step(bt->d_group, bt->group_blocks, o.precision, dt, n, bt->group_block, s);
+      int e = bt->group_trees ? launch_grouped_trees(bt->d_group, bt->group_blocks, bt->group_lds, o.precision, dt, n,
+                                                     bt->group_block, s)
+                              : launch_grouped_step(bt->d_group, bt->group_blocks, o.precision, dt, n, bt->group_block, s);
       if (e) return fail(GP_ERR_DEVICE, "grouped kernel launch: %s", hipGetErrorString((hipError_t)e));
       ++*launches;
     }
@@ -636,7 +688,7 @@ static int batch_launch_all(gp_batch* bt, double dt, int integrator, int n_steps
     bool fast = bucket_is_fast(o, b, integrator);
     if (o.kernel == GP_KERNEL_FAST && !fast)
       return fail(GP_ERR_UNSUPPORTED, "no FAST kernel for this bucket's topology / integrator");
-    if (fast && grouped) continue;
+    if (grouped && in_group(o, b, integrator, bt->group_trees)) continue;
     if (is_velocity_stepping(integrator)) {
       if (o.precision == GP_PREC_MIXED && o.kernel == GP_KERNEL_PLAIN)
         return fail(GP_ERR_UNSUPPORTED, "velocity stepping computes in FP64 only");
@@ -677,6 +729,14 @@ static int batch_launch_all(gp_batch* bt, double dt, int integrator, int n_steps
                     ? launch_fast_step(b.fast_topo, o.precision, a, dt, n, o.block_size, s)
                     : launch_fast_rk_step(b.fast_topo, o.precision, integrator, a, dt, n, o.block_size, s);
         if (e) return fail(GP_ERR_DEVICE, "fast kernel launch: %s", hipGetErrorString((hipError_t)e));
+        ++*launches;
+      }
+    } else if (bucket_aux_tree(o, b, integrator)) {
+      const int spl = o.steps_per_launch > 0 ? o.steps_per_launch : 100;
+      BucketArgs a = bucket_args(b, b.nb, nullptr);
+      for (int done = 0; done < n_steps; done += spl) {
+        int e = launch_fast_step(TOPO_TREE, GP_PREC_F64, a, dt, std::min(spl, n_steps - done), o.block_size, s);
+        if (e) return fail(GP_ERR_DEVICE, "tree kernel launch: %s", hipGetErrorString((hipError_t)e));
         ++*launches;
       }
     } else {

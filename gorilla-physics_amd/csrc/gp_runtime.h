@@ -48,6 +48,8 @@ struct Bucket {
   std::vector<int64_t> inst;  // lane -> instance index
   int *d_parent = nullptr, *d_qoff = nullptr, *d_voff = nullptr, *d_cstart = nullptr, *d_kind = nullptr;
   int* d_sstart = nullptr;
+  int *d_depth = nullptr, *d_child_start = nullptr, *d_child = nullptr;
+  int max_depth = 0;
   double *d_sp = nullptr, *d_ss = nullptr;
   int* d_sphere_of = nullptr;
   double* d_shp = nullptr;
@@ -86,6 +88,8 @@ struct Bucket {
       o.d_rounds = nullptr;
       d_active = o.d_active; d_scratch = o.d_scratch; d_arena = o.d_arena; arena_bytes = o.arena_bytes;
       d_flat_off = o.d_flat_off;
+      d_depth = o.d_depth; d_child_start = o.d_child_start; d_child = o.d_child; max_depth = o.max_depth;
+      o.d_depth = o.d_child_start = o.d_child = nullptr;
       o.d_arena = nullptr;
       o.d_flat_off = nullptr;
       o.d_parent = o.d_qoff = o.d_voff = o.d_cstart = o.d_kind = o.d_fault = o.d_active = nullptr;
@@ -132,6 +136,8 @@ struct gp_batch {
   gp::GroupTable* d_group = nullptr;
   int group_blocks = 0, group_block = 0;
   bool group_valid = false;
+  bool group_trees = false;  // every bucket of the group is a tree (launch_grouped_trees)
+  int group_lds = 0;         // its LDS bytes per wave
   // device tables of the transfers between flat device arrays and the buckets:
   // state (q and v), torques, accelerations, each one launch
   struct Xfer { int at = 0, n = 0; unsigned blocks = 0; };

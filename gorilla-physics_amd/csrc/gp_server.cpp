@@ -292,7 +292,7 @@ int rebuild_group(gp_server* s) {
     t.args[t.n] = a;
     t.topo[t.n] = p.b.fast_topo;
     t.block_start[t.n] = blocks.back();
-    blocks.back() += (int)(((int64_t)p.b.B * lanes + block - 1) / block);
+    blocks.back() += (int)((fast_threads(p.b.fast_topo, p.b.B, lanes) + block - 1) / block);
     ++t.n;
     t.block_start[t.n] = blocks.back();
   }

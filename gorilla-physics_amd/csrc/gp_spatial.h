@@ -119,6 +119,10 @@ struct ai6 {
   m3<R> B;
   s3<R> C;
 };
+template <class D, class S> GP_HD ai6<D> cvt(const ai6<S>& I) {
+  return {{D(I.A.xx), D(I.A.yy), D(I.A.zz), D(I.A.xy), D(I.A.xz), D(I.A.yz)}, cvt<D>(I.B),
+          {D(I.C.xx), D(I.C.yy), D(I.C.zz), D(I.C.xy), D(I.C.xz), D(I.C.yz)}};
+}
 template <class R> GP_HD sv<R> mul(const ai6<R>& I, const sv<R>& m) {
   return {mul(I.A, m.w) + mul(I.B, m.v), mulT(I.B, m.w) + mul(I.C, m.v)};
 }

@@ -1,23 +1,32 @@
-// gp_tree_impl.h — trees of many bodies, one instance per L lanes (L = 16, 32
-// or 64, at least the body count), lane j of an instance holding body j and
-// its joint. The articulated-body algorithm (RBDA Table 7.1) runs its three
-// sweeps level by level: every body of one depth at once, a body's parent
-// quantities (velocity, world pose, acceleration) taken from the parent's
-// lane by a cross-lane shuffle on the way out, and on the way in each parent
-// summing its children's articulated inertias and bias forces by reading them
-// from the children's lanes. The lanes exchange through LDS: each lane has a
-// slot of kTreeSlot doubles, written by the lane when its level is done and
-// read by its children (pass 1 and 3) or its parent (pass 2) one level later;
-// all lanes of a segment are in one wave, whose LDS instructions execute in
-// order, so no barrier is needed, only a compiler fence between levels. Runtime
-// topology: any tree of up to 64 bodies with at most kTreeMaxChildren
-// children per body, every joint type, contact points, prismatic springs;
-// semi-implicit Euler (integrators.rs:276-319), n_steps steps per launch with
-// each lane's joint state, parameters and per-body quantities in registers.
-// The joint accelerations are those of the reference's dynamics_continuous
+// gp_tree_impl.h — trees of bodies, one body and its joint per lane: an
+// instance takes as many neighbouring lanes of one wave as it has bodies, and
+// a wave holds as many whole instances as fit in its 64 lanes (three hexapods
+// of 19 bodies, seven quadrupeds of 9). The articulated-body algorithm (RBDA
+// Table 7.1) runs its three sweeps level by level: every body of one depth at
+// once, each reading its parent's velocity, world pose or acceleration on the
+// way out and its children's articulated inertias and bias forces on the way
+// in. The lanes exchange through LDS: each lane has a slot of kTreeSlot
+// doubles, written by the lane when its level is done and read by its children
+// (pass 1 and 3) or its parent (pass 2) one level later; all lanes of an
+// instance are in one wave, whose LDS instructions execute in order, so no
+// barrier is needed, only a compiler fence between levels. Runtime topology:
+// any tree of up to 64 bodies with at most kTreeMaxChildren children per
+// body, every joint type, contact points, prismatic springs; semi-implicit
+// Euler (integrators.rs:276-319), n_steps steps per launch. The joint
+// accelerations are those of the reference's dynamics_continuous
 // (dynamics.rs:322-364). R = double: FP64 throughout; R = float: FP32 sweeps,
 // FP64 joint-space solves, contact distances and q/v (as the other mixed
 // kernels).
+//
+// What bounds it: each level's instructions issue for the whole wave with the
+// other depths' lanes masked off, and each level waits for the one before
+// through LDS. So: instances packed by their body count, not by a power of two
+// above it, and two waves per SIMD, which 256 registers a lane allow once a
+// floating joint's coordinates (one lane in a tree has them) live in LDS
+// instead of every lane's registers. Measured with the state's transfers on
+// one MI355X, ten steps: 8,191 trees of 16-40 bodies 1,060 -> 534 us (one wave
+// per SIMD, two instances a wave before); 2,048 nine-body quadrupeds with
+// twelve foot contacts 986 (plain kernel) -> 122 us.
 // Included by gp_fast_impl.h (it uses Soa, pick and joint_frame from there).
 #pragma once
 
@@ -27,7 +36,6 @@ constexpr int kTreeMaxChildren = 8;
 // doubles per lane in the exchange slot (an articulated inertia and a force,
 // 21 + 6; odd, so a wave's 64-bit accesses spread over the banks)
 constexpr int kTreeSlot = 27;
-constexpr int kTreeSlotBytes = kTreeSlot * 8;
 
 // slot <-> spatial vector / articulated inertia, in the sweeps' precision R
 // from the slot's start (the slot is a row of doubles)
@@ -54,16 +62,20 @@ template <class R> __device__ __forceinline__ ai6<R> get_ai6(const R* p) {
 // a compiler-only barrier between levels: slot reads are not moved above the
 // writes of the level before (the hardware keeps one wave's LDS order)
 __device__ __forceinline__ void level_fence() { asm volatile("" ::: "memory"); }
-template <int L> __device__ __forceinline__ int seg_max(int x) {
-#pragma unroll
-  for (int off = 1; off < L; off <<= 1) x = max(x, __shfl_xor(x, off, L));
-  return x;
-}
 
-// Whether a bucket's topology runs on this kernel: more bodies than the
-// compiled chains, at most 64, no body with more than kTreeMaxChildren children.
+// doubles of a floating joint's coordinates in LDS: q, v, torques, accelerations
+constexpr int kTreeFloat = 7 + 6 + 6 + 6;
+// most LDS a lane can account for (a floating body alone)
+constexpr int kTreeLaneBytes = (kTreeSlot + kTreeFloat) * 8;
+// LDS doubles of an instance: its bodies' slots, then its floating joints
+inline __host__ __device__ int tree_seg_doubles(int nb, int floating) { return kTreeSlot * nb + kTreeFloat * floating; }
+// LDS bytes of one wave
+inline int tree_wave_bytes(int nb, int floating) { return 64 / nb * tree_seg_doubles(nb, floating) * 8; }
+
+// Whether a topology runs on this kernel: at most 64 bodies, none with more
+// than kTreeMaxChildren children.
 inline bool tree_topology_ok(int nb, const int* parent) {
-  if (nb < 13 || nb > 64) return false;
+  if (nb < 1 || nb > 64) return false;
   for (int i = 0; i < nb; ++i) {
     int c = 0;
     for (int k = i + 1; k < nb; ++k) c += parent[k] == i ? 1 : 0;
@@ -71,13 +83,60 @@ inline bool tree_topology_ok(int nb, const int* parent) {
   }
   return true;
 }
-inline int tree_lanes(int nb) { return nb <= 16 ? 16 : nb <= 32 ? 32 : 64; }
 
-template <class R, int L>
+// L^T D L of a floating joint's 6x6 inertia, packed by rows: unit lower factor
+// below the diagonal, reciprocal pivots on it; false if a pivot is not positive.
+__device__ __forceinline__ bool ldl6(const ai6<double>& I, double (&L)[21]) {
+  L[0] = I.A.xx;
+  L[1] = I.A.xy; L[2] = I.A.yy;
+  L[3] = I.A.xz; L[4] = I.A.yz; L[5] = I.A.zz;
+#pragma unroll
+  for (int r = 0; r < 3; ++r)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) L[(3 + r) * (4 + r) / 2 + c] = I.B.a[3 * c + r];
+  L[9] = I.C.xx;
+  L[13] = I.C.xy; L[14] = I.C.yy;
+  L[18] = I.C.xz; L[19] = I.C.yz; L[20] = I.C.zz;
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < 6; ++j) {
+    // column j below the pivot still holds L_ij d_j of the columns before
+    const int jj = j * (j + 1) / 2;
+    ok = ok && (L[jj + j] > 0.0);
+    const double inv = recip(L[jj + j]);
+#pragma unroll
+    for (int i = j + 1; i < 6; ++i) {
+      const int ii = i * (i + 1) / 2;
+      const double lij = L[ii + j] * inv;
+#pragma unroll
+      for (int k = j + 1; k <= i; ++k) L[ii + k] -= lij * L[k * (k + 1) / 2 + j];
+    }
+#pragma unroll
+    for (int i = j + 1; i < 6; ++i) L[i * (i + 1) / 2 + j] *= inv;
+    L[jj + j] = inv;
+  }
+  return ok;
+}
+__device__ __forceinline__ void ldl6_solve(const double (&L)[21], double (&x)[6]) {
+#pragma unroll
+  for (int i = 1; i < 6; ++i)
+#pragma unroll
+    for (int k = 0; k < i; ++k) x[i] -= L[i * (i + 1) / 2 + k] * x[k];
+#pragma unroll
+  for (int i = 0; i < 6; ++i) x[i] *= L[i * (i + 1) / 2 + i];
+#pragma unroll
+  for (int i = 4; i >= 0; --i)
+#pragma unroll
+    for (int k = i + 1; k < 6; ++k) x[i] -= L[k * (k + 1) / 2 + i] * x[k];
+}
+
+template <class R>
 __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, double dt, int n_steps) {
-  const int inst = tid / L, j = tid % L;
-  if (inst >= a.B) return;  // the whole L-lane segment leaves together
   const int nb = a.nb, Bp = a.Bp;
+  const int ipw = 64 / nb;  // instances per wave
+  const int w = tid & 63, seg = w / nb, j = w - seg * nb;
+  const int inst = (tid >> 6) * ipw + seg;
+  if (seg >= ipw || inst >= a.B) return;  // an instance's lanes leave together
   int my_steps = n_steps;
   if (a.active) {  // serving: the instance's remaining horizon
     const int left = a.active[inst];
@@ -85,99 +144,86 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
     my_steps = min(my_steps, left);
     if (j == 0) a.active[inst] = left - my_steps;
   }
-  const bool live = j < nb;
-  // ---- topology of this lane's body
-  const int par = live ? a.parent[j] : -1;
-  // exchange slots: the segment's (its lane 0 is block lane threadIdx.x - j,
-  // blockDim being a multiple of L) and this lane's
-  double* const seg = (double*)GP_DYN_LDS + (size_t)((int)threadIdx.x - j) * kTreeSlot;
-  double* const mine = seg + j * kTreeSlot;
-  R* const mineR = (R*)mine;
-  int depth = -1;
-  if (live) {
-    depth = 0;
-    for (int k = par; k >= 0; k = a.parent[k]) ++depth;
-  }
-  const int maxd = seg_max<L>(depth);
-  int child[kTreeMaxChildren];
-  int nch = 0;
-#pragma unroll
-  for (int k = 0; k < kTreeMaxChildren; ++k) child[k] = j;
-  if (live)
-    for (int k = j + 1; k < nb; ++k)
-      if (a.parent[k] == j && nch < kTreeMaxChildren) child[nch++] = k;
-  const int maxc = seg_max<L>(nch);
+  // ---- topology of this lane's body (tables built by the host)
+  const int maxd = a.max_depth;
+  const int par = a.parent[j], depth = a.depth[j];
+  const int ch0 = a.child_start[j], nch = a.child_start[j + 1] - ch0;
+  unsigned long long child = 0;  // the children's lanes, a byte each
+  for (int k = 0; k < nch; ++k) child |= (unsigned long long)a.child[ch0 + k] << (8 * k);
+  const int qo = a.qoff[j], vo = a.voff[j];
   const Soa<int> kindS(a.kind, nb, Bp);
-  const int kind = live ? kindS.ld(j, inst) : K_FIXED;
-  const int qo = live ? a.qoff[j] : 0, vo = live ? a.voff[j] : 0;
-  const int nqj = kind == K_FLOAT ? 7 : (kind == K_FIXED ? 0 : 1);
-  const int nvj = kind == K_FLOAT ? 6 : (kind == K_FIXED ? 0 : 1);
+  const int kind = kindS.ldx(0, inst, j);
+  const bool one = kind == K_REV || kind == K_PRI;
+  // exchange slots: the instance's and this lane's; then its floating joints'
+  // coordinates (one more q than v each, so qo - vo numbers them)
+  double* const lds = (double*)GP_DYN_LDS + ((size_t)(threadIdx.x >> 6) * ipw + seg) * tree_seg_doubles(nb, a.nq - a.nv);
+  double* const mine = lds + j * kTreeSlot;
+  R* const mineR = (R*)mine;
+  double* const fl = lds + nb * kTreeSlot + (qo - vo) * kTreeFloat;
   // ---- parameters and state of this lane's body and joint, for the launch
   const Soa<double> bpS(a.bp, NBF * nb, Bp);
   const Soa<R> bpR(pick<R>(a.bp, a.bpf), NBF * nb, Bp);
-  const int jb = live ? j : 0;
+  auto pd = [&](int f) { return bpS.ldx(f * nb, inst, j); };
+  auto pr = [&](int f) { return bpR.ldx(f * nb, inst, j); };
   m3<double> Rt;
-  v3<double> pt;
 #pragma unroll
-  for (int k = 0; k < 9; ++k) Rt.a[k] = bpS.ld((BF_RT + k) * nb + jb, inst);
-  pt = v3<double>{bpS.ld(BF_PT * nb + jb, inst), bpS.ld((BF_PT + 1) * nb + jb, inst), bpS.ld((BF_PT + 2) * nb + jb, inst)};
-  const m3<R> RtR = cvt<R>(Rt);
-  const v3<R> ptR = cvt<R>(pt);
-  const s3<R> J{bpR.ld(BF_J * nb + jb, inst), bpR.ld((BF_J + 1) * nb + jb, inst), bpR.ld((BF_J + 2) * nb + jb, inst),
-                bpR.ld((BF_J + 3) * nb + jb, inst), bpR.ld((BF_J + 4) * nb + jb, inst),
-                bpR.ld((BF_J + 5) * nb + jb, inst)};
-  const v3<R> mc{bpR.ld(BF_C * nb + jb, inst), bpR.ld((BF_C + 1) * nb + jb, inst), bpR.ld((BF_C + 2) * nb + jb, inst)};
-  const R mass = bpR.ld(BF_M * nb + jb, inst);
-  const double sk = kind == K_PRI ? bpS.ld(BF_SK * nb + jb, inst) : 0.0;
-  const double sl = kind == K_PRI ? bpS.ld(BF_SL * nb + jb, inst) : 0.0;
+  for (int k = 0; k < 9; ++k) Rt.a[k] = pd(BF_RT + k);
+  const v3<double> pt{pd(BF_PT), pd(BF_PT + 1), pd(BF_PT + 2)};
+  const s3<R> J{pr(BF_J), pr(BF_J + 1), pr(BF_J + 2), pr(BF_J + 3), pr(BF_J + 4), pr(BF_J + 5)};
+  const v3<R> mc{pr(BF_C), pr(BF_C + 1), pr(BF_C + 2)};
+  const R mass = pr(BF_M);
+  const double sk = kind == K_PRI ? pd(BF_SK) : 0.0;
+  const double sl = kind == K_PRI ? pd(BF_SL) : 0.0;
   const Soa<double> qS(a.q, a.nq, Bp), vS(a.v, a.nv, Bp), tauS(a.tau, a.nv, Bp), vdotS(a.vdot, a.nv, Bp);
   const Soa<double> cpS(a.cp, NCF * a.nc, Bp), hpS(a.hp, NHF * a.nh, Bp);
-  double q[7], v[6], tau[6], vd[6];
+  double q = 0.0, v = 0.0, tau = 0.0, vd = 0.0;  // of a one-DOF joint
+  if (one) {
+    q = qS.ldx(0, inst, qo);
+    v = vS.ldx(0, inst, vo);
+    tau = tauS.ldx(0, inst, vo);
+  } else if (kind == K_FLOAT) {
 #pragma unroll
-  for (int k = 0; k < 7; ++k) q[k] = k < nqj ? qS.ldx(0, inst, qo + k) : 0.0;
+    for (int k = 0; k < 7; ++k) fl[k] = qS.ldx(k, inst, qo);
 #pragma unroll
-  for (int k = 0; k < 6; ++k) {
-    v[k] = k < nvj ? vS.ldx(0, inst, vo + k) : 0.0;
-    tau[k] = k < nvj ? tauS.ldx(0, inst, vo + k) : 0.0;
-    vd[k] = 0.0;
+    for (int k = 0; k < 6; ++k) {
+      fl[7 + k] = vS.ldx(k, inst, vo);
+      fl[13 + k] = tauS.ldx(k, inst, vo);
+    }
   }
   const bool contacts = a.nc > 0;
-  const int c0 = live ? a.cstart[j] : 0, c1 = live ? a.cstart[j + 1] : 0;
+  const int c0 = a.cstart[j], c1 = a.cstart[j + 1];
   bool ok = true;
-  const ai6<R> I = rigid(J, mc, mass);
   for (int s = 0; s < my_steps; ++s) {
     // ---- this joint's transform (E, r: parent -> body) and velocity S qd
     m3<R> E;
     v3<R> r;
-    m3<double> Rm_d;  // body -> parent rotation and translation, FP64 (contacts, floating pose)
-    v3<double> p_d;
     sv<R> vj{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
+    m3<double> Rw;  // body -> parent, then world: rotation and translation, FP64 (contacts, floating pose)
+    v3<double> tw;
     if (kind == K_FLOAT) {
-      Rm_d = mul(Rt, quat_mat(q[0], q[1], q[2], q[3]));
-      p_d = pt + mul(Rt, v3<double>{q[4], q[5], q[6]});
-      const m3<R> Rm = cvt<R>(Rm_d);
+      Rw = mul(Rt, quat_mat(fl[0], fl[1], fl[2], fl[3]));
+      tw = pt + mul(Rt, v3<double>{fl[4], fl[5], fl[6]});
+      const m3<R> Rm = cvt<R>(Rw);
       E = m3<R>{{Rm.a[0], Rm.a[3], Rm.a[6], Rm.a[1], Rm.a[4], Rm.a[7], Rm.a[2], Rm.a[5], Rm.a[8]}};
-      r = cvt<R>(p_d);
-      vj = sv<R>{{R(v[0]), R(v[1]), R(v[2])}, {R(v[3]), R(v[4]), R(v[5])}};
+      r = cvt<R>(tw);
+      vj = sv<R>{{R(fl[7]), R(fl[8]), R(fl[9])}, {R(fl[10]), R(fl[11]), R(fl[12])}};
     } else {
       R cs = R(1), sn = R(0), dd = R(0);
-      if (kind == K_REV) sincos_q(q[0], &sn, &cs);
-      if (kind == K_PRI) dd = R(q[0]);
-      joint_frame(RtR, ptR, cs, sn, dd, E, r);
-      if (kind == K_REV) vj.w.z = R(v[0]);
-      if (kind == K_PRI) vj.v.z = R(v[0]);
+      if (kind == K_REV) sincos_q(q, &sn, &cs);
+      if (kind == K_PRI) dd = R(q);
+      joint_frame(cvt<R>(Rt), cvt<R>(pt), cs, sn, dd, E, r);
+      if (kind == K_REV) vj.w.z = R(v);
+      if (kind == K_PRI) vj.v.z = R(v);
       if (contacts) {
         const m3<double> Ed = cvt<double>(E);
-        Rm_d = m3<double>{{Ed.a[0], Ed.a[3], Ed.a[6], Ed.a[1], Ed.a[4], Ed.a[7], Ed.a[2], Ed.a[5], Ed.a[8]}};
-        p_d = cvt<double>(r);
+        Rw = m3<double>{{Ed.a[0], Ed.a[3], Ed.a[6], Ed.a[1], Ed.a[4], Ed.a[7], Ed.a[2], Ed.a[5], Ed.a[8]}};
+        tw = cvt<double>(r);
       }
     }
     // ---- pass 1, root to leaves by depth: velocities (and world poses);
     // slot: velocity (R) from the start, world rotation doubles [6, 15),
     // world translation doubles [15, 18)
     sv<R> vel = vj;
-    m3<double> Rw = Rm_d;
-    v3<double> tw = p_d;
     auto put_pose = [&]() {
       put_sv(mineR, vel);
       if (contacts) {
@@ -191,21 +237,27 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
     for (int d = 1; d <= maxd; ++d) {
       level_fence();
       if (depth == d) {
-        const double* ps = seg + par * kTreeSlot;
+        const double* ps = lds + par * kTreeSlot;
         vel = xmotion(E, r, get_sv<R>((const R*)ps)) + vj;
         if (contacts) {
           m3<double> pR;
 #pragma unroll
           for (int k = 0; k < 9; ++k) pR.a[k] = ps[6 + k];
-          tw = v3<double>{ps[15], ps[16], ps[17]} + mul(pR, p_d);
-          Rw = mul(pR, Rm_d);
+          tw = v3<double>{ps[15], ps[16], ps[17]} + mul(pR, tw);
+          Rw = mul(pR, Rw);
         }
         if (d < maxd) put_pose();
       }
     }
     // velocity-product acceleration, rigid-body bias force, contact forces
     const sv<R> cb = crm(vel, vj);
-    sv<R> pA = crf(vel, mul(I, vel));
+    const ai6<R> I = rigid(J, mc, mass);
+    sv<R> pA;
+    {
+      // v x* (I v): w x (J w) + c x g and m g + w x (w x c) with g = w x v
+      const v3<R> g = cross(vel.w, vel.v), hw = mul(J, vel.w), wc = cross(vel.w, mc);
+      pA = sv<R>{cross(vel.w, hw) + cross(mc, g), mass * g + cross(vel.w, wc)};
+    }
     if (contacts && c0 < c1) {
       const m3<R> RwR = cvt<R>(Rw);
       sv<R> fe{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
@@ -216,7 +268,7 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
         const double off = dot(tw - v3<double>{hpar(HF_POINT), hpar(HF_POINT + 1), hpar(HF_POINT + 2)}, n);
         const R alpha = R(hpar(HF_ALPHA)), mu = R(hpar(HF_MU));
         for (int cc = c0; cc < c1; ++cc) {
-          auto cpar = [&](int fld) { return cpS.ld(fld * a.nc + cc, inst); };
+          auto cpar = [&](int fld) { return cpS.ldx(fld * a.nc, inst, cc); };
           const v3<double> pb{cpar(CF_P), cpar(CF_P + 1), cpar(CF_P + 2)};
           const double dist = dot(nb_, pb) + off;
           if (dist <= kInsideMargin) {
@@ -234,135 +286,143 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
     // ---- pass 2, leaves to root by depth: articulated inertias and bias forces
     ai6<R> IA = I;
     sv<R> U{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
-    double Dinv = 0.0, u = 0.0, u6[6] = {0, 0, 0, 0, 0, 0};
-    for (int d = maxd; d >= 0; --d) {
-      ai6<R> cI{};
-      sv<R> cf{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
+    double Dinv = 0.0, u = 0.0;
+    // a one-DOF joint's U, D and u (tq: torque and prismatic spring, dynamics.rs:298-315)
+    auto solve_one = [&]() {
+      const bool rev = kind == K_REV;
+      U = rev ? col(IA, 2) : col(IA, 5);
+      Dinv = recip(double(rev ? IA.A.zz : IA.C.zz));
+      ok = ok && (Dinv > 0.0);
+      const double tq = tau - sk * (q - sl);
+      u = tq - double(rev ? pA.w.z : pA.v.z);
+    };
+    for (int d = maxd; d >= 1; --d) {
       if (depth == d) {
-        ai6<R> Ia = IA;
-        sv<R> pa = pA + mul(IA, cb);
-        if (kind == K_REV || kind == K_PRI) {
-          const bool rev = kind == K_REV;
-          U = rev ? col(IA, 2) : col(IA, 5);
-          Dinv = 1.0 / double(rev ? IA.A.zz : IA.C.zz);
-          const double tq = tau[0] - sk * (q[0] - sl);  // prismatic spring (dynamics.rs:298-315); 0 otherwise
-          u = tq - double(rev ? pA.w.z : pA.v.z);
-          ok = ok && (Dinv > 0.0);
+        // in place: IA becomes the joint's Ia
+        sv<R> pa;
+        if (one) {
+          solve_one();
           const R inv = R(Dinv);
           const sv<R> uD{inv * U.w, inv * U.v};
-          Ia = rank1_down(IA, U, uD);
+          IA = rank1_down(IA, U, uD);
           const R uR = R(u);
-          pa = pA + mul(Ia, cb) + sv<R>{uR * uD.w, uR * uD.v};
+          pa = pA + mul(IA, cb) + sv<R>{uR * uD.w, uR * uD.v};
         } else if (kind == K_FLOAT) {
-          u6[0] = tau[0] - double(pA.w.x); u6[1] = tau[1] - double(pA.w.y); u6[2] = tau[2] - double(pA.w.z);
-          u6[3] = tau[3] - double(pA.v.x); u6[4] = tau[4] - double(pA.v.y); u6[5] = tau[5] - double(pA.v.z);
-          Ia = ai6<R>{};  // I^A - I^A (I^A)^-1 I^A = 0
-          pa = pA + sv<R>{{R(u6[0]), R(u6[1]), R(u6[2])}, {R(u6[3]), R(u6[4]), R(u6[5])}};
+          // Ia = I^A - I^A (I^A)^-1 I^A = 0 (IA stays for pass 3); pA + u is the whole torque
+#pragma unroll
+          for (int k = 0; k < 21; ++k) mineR[k] = R(0);
+          pa = sv<R>{{R(fl[13]), R(fl[14]), R(fl[15])}, {R(fl[16]), R(fl[17]), R(fl[18])}};
+        } else {
+          pa = pA + mul(IA, cb);
         }
-        cI = xtix(E, r, Ia);
-        cf = xtforce(E, r, pa);
-        if (d > 0) {  // slot (R): articulated inertia [0, 21), bias force [21, 27)
-          put_ai6(mineR, cI);
-          put_sv(mineR + 21, cf);
-        }
+        // slot (R): articulated inertia [0, 21), bias force [21, 27)
+        if (kind != K_FLOAT) put_ai6(mineR, xtix(E, r, IA));
+        put_sv(mineR + 21, xtforce(E, r, pa));
       }
-      if (d == 0) break;
       // parents (depth d - 1) take their children's parts, in child order
       level_fence();
       if (depth == d - 1) {
-#pragma unroll
-        for (int k = 0; k < kTreeMaxChildren; ++k) {
-          if (k < nch) {
-            const R* cs = (const R*)(seg + child[k] * kTreeSlot);
-            add_to(IA, get_ai6<R>(cs));
-            pA = pA + get_sv<R>(cs + 21);
-          }
+        for (int k = 0; k < nch; ++k) {
+          const R* cs = (const R*)(lds + (int)((child >> (8 * k)) & 63) * kTreeSlot);
+          add_to(IA, get_ai6<R>(cs));
+          pA = pA + get_sv<R>(cs + 21);
         }
       }
       level_fence();  // the slots read here are written again only in pass 3
     }
+    if (depth == 0 && one) solve_one();
     // ---- pass 3, root to leaves by depth: accelerations, then the joint's step
-    sv<R> acc{{R(0), R(0), R(0)}, {R(0), R(0), R(a.g)}};  // gravity as the base's acceleration
     for (int d = 0; d <= maxd; ++d) {
       level_fence();
       if (depth == d) {
-        const sv<R> pacc = par < 0 ? sv<R>{{R(0), R(0), R(0)}, {R(0), R(0), R(a.g)}} : get_sv<R>((const R*)(seg + par * kTreeSlot));
+        sv<R> pacc{{R(0), R(0), R(0)}, {R(0), R(0), R(a.g)}};  // gravity as the base's acceleration
+        if (d > 0) pacc = get_sv<R>((const R*)(lds + par * kTreeSlot));
         sv<R> ap = xmotion(E, r, pacc) + cb;
-        if (kind == K_REV || kind == K_PRI) {
+        if (one) {
           const double qdd = (u - double(dot6(U, ap))) * Dinv;
-          vd[0] = qdd;
+          vd = qdd;
           if (kind == K_REV) ap.w.z += R(qdd);
           else ap.v.z += R(qdd);
         } else if (kind == K_FLOAT) {
-          double D6[6][6], Lf[21];
-          to_dense(IA, D6);
-          ok = chol6(D6, Lf) && ok;
-          const double apd[6] = {double(ap.w.x), double(ap.w.y), double(ap.w.z),
-                                 double(ap.v.x), double(ap.v.y), double(ap.v.z)};
-          double x[6];
+          const ai6<double> Id = cvt<double>(IA);
+          const sv<double> apd{cvt<double>(ap.w), cvt<double>(ap.v)}, pAd{cvt<double>(pA.w), cvt<double>(pA.v)};
+          const sv<double> Ia = mul(Id, apd);
+          double L[21];
+          double x[6] = {fl[13] - pAd.w.x - Ia.w.x, fl[14] - pAd.w.y - Ia.w.y, fl[15] - pAd.w.z - Ia.w.z,
+                         fl[16] - pAd.v.x - Ia.v.x, fl[17] - pAd.v.y - Ia.v.y, fl[18] - pAd.v.z - Ia.v.z};
+          ok = ldl6(Id, L) && ok;
+          ldl6_solve(L, x);
 #pragma unroll
-          for (int rr = 0; rr < 6; ++rr) {
-            double t = u6[rr];
-#pragma unroll
-            for (int cc = 0; cc < 6; ++cc) t -= D6[rr][cc] * apd[cc];
-            x[rr] = t;
-          }
-          chol6_solve(Lf, x);
-#pragma unroll
-          for (int t = 0; t < 6; ++t) vd[t] = x[t];
+          for (int t = 0; t < 6; ++t) fl[19 + t] = x[t];
           ap = ap + sv<R>{{R(x[0]), R(x[1]), R(x[2])}, {R(x[3]), R(x[4]), R(x[5])}};
         }
-        acc = ap;
-        if (d < maxd) put_sv(mineR, acc);  // slot (R): acceleration from the start
+        if (d < maxd) put_sv(mineR, ap);  // slot (R): acceleration from the start
       }
     }
-    // ---- semi-implicit Euler of this lane's joint (integrators.rs:276-319)
+    // ---- semi-implicit Euler of this lane's joint (integrators.rs:276-319); a
+    // non-finite acceleration leaves v non-finite for good
+    if (kind == K_FLOAT) {
+      double qf[7], vf[6];
+#pragma unroll
+      for (int k = 0; k < 7; ++k) qf[k] = fl[k];
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        vf[k] = fl[7 + k] + fl[19 + k] * dt;
+        fl[7 + k] = vf[k];
+      }
+      advance_floating(qf, vf, dt, qf);
+#pragma unroll
+      for (int k = 0; k < 7; ++k) fl[k] = qf[k];
+    } else if (one) {
+      v = v + vd * dt;
+      q += v * dt;
+    }
+  }
+  if (one) {
+    qS.stx(0, inst, qo, q);
+    vS.stx(0, inst, vo, v);
+    vdotS.stx(0, inst, vo, vd);
+    ok = ok && isfinite(q) && isfinite(v);
+  } else if (kind == K_FLOAT) {
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+      const double x = fl[k];
+      qS.stx(k, inst, qo, x);
+      ok = ok && isfinite(x);
+    }
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      if (k < nvj) ok = ok && isfinite(vd[k]);
-      v[k] = v[k] + vd[k] * dt;
+      const double x = fl[7 + k];
+      vS.stx(k, inst, vo, x);
+      vdotS.stx(k, inst, vo, fl[19 + k]);
+      ok = ok && isfinite(x);
     }
-    if (kind == K_FLOAT) advance_floating(q, v, dt, q);
-    else q[0] += v[0] * dt;
   }
-  if (live) {
-#pragma unroll
-    for (int k = 0; k < 7; ++k)
-      if (k < nqj) {
-        qS.stx(0, inst, qo + k, q[k]);
-        ok = ok && isfinite(q[k]);
-      }
-#pragma unroll
-    for (int k = 0; k < 6; ++k)
-      if (k < nvj) {
-        vS.stx(0, inst, vo + k, v[k]);
-        vdotS.stx(0, inst, vo + k, vd[k]);
-        ok = ok && isfinite(v[k]);
-      }
-  }
-  // any lane's fault is the instance's
-  int bad = ok ? 0 : 1;
-#pragma unroll
-  for (int off = 1; off < L; off <<= 1) bad |= __shfl_xor(bad, off, L);
-  if (j == 0 && bad) a.fault[inst] = 1;
+  if (!ok) a.fault[inst] = 1;  // any lane's fault is the instance's
 }
 
-template <class R, int L>
-__global__ void __launch_bounds__(256) wave_tree_kernel(BucketArgs a, double dt, int n_steps) {
-  wave_tree_body<R, L>(a, blockIdx.x * blockDim.x + threadIdx.x, dt, n_steps);
+// Two waves per SIMD (at most 256 registers a lane)
+template <class R>
+__global__ void __launch_bounds__(256, 2) wave_tree_kernel(BucketArgs a, double dt, int n_steps) {
+  wave_tree_body<R>(a, blockIdx.x * blockDim.x + threadIdx.x, dt, n_steps);
+}
+// Every bucket of a batch of trees in one launch, at the occupancy of the
+// kernel above (the grouped launch over all compiled topologies runs at one
+// wave per SIMD).
+template <class R>
+__global__ void __launch_bounds__(256, 2) grouped_tree_kernel(const GroupTable* __restrict__ t, double dt, int n_steps) {
+  int b = 0;
+  while (b + 1 < t->n && (int)blockIdx.x >= t->block_start[b + 1]) ++b;  // uniform per workgroup
+  const BucketArgs a = t->args[b];
+  const int tid = ((int)blockIdx.x - t->block_start[b]) * (int)blockDim.x + (int)threadIdx.x;
+  wave_tree_body<R>(a, tid, dt, n_steps);
 }
 
 template <class R>
 static int launch_wave_tree(const BucketArgs& a, double dt, int n_steps, int block, hipStream_t s) {
-  const long threads = (long)a.B * a.lanes;
-  dim3 blk(block), grid((unsigned)((threads + block - 1) / block));
-  const unsigned lds = (unsigned)(kTreeSlotBytes * block);
-  switch (a.lanes) {
-    case 16: hipLaunchKernelGGL((wave_tree_kernel<R, 16>), grid, blk, lds, s, a, dt, n_steps); break;
-    case 32: hipLaunchKernelGGL((wave_tree_kernel<R, 32>), grid, blk, lds, s, a, dt, n_steps); break;
-    case 64: hipLaunchKernelGGL((wave_tree_kernel<R, 64>), grid, blk, lds, s, a, dt, n_steps); break;
-    default: return (int)hipErrorInvalidValue;
-  }
+  dim3 blk(block), grid((unsigned)((fast_threads(TOPO_TREE, a.B, a.nb) + block - 1) / block));
+  const unsigned lds = (unsigned)(block / 64 * tree_wave_bytes(a.nb, a.nq - a.nv));
+  hipLaunchKernelGGL((wave_tree_kernel<R>), grid, blk, lds, s, a, dt, n_steps);
   return (int)hipGetLastError();
 }
 

@@ -83,6 +83,9 @@ enum {
 /* ---- kernel family --------------------------------------------------------- */
 enum {
   GP_KERNEL_AUTO = 0,  /* FAST when the bucket topology has a compiled kernel;
+                          semi-implicit Euler of any other tree without spring
+                          contacts and with at most 8 children a body: one
+                          body per lane, FP64;
                           velocity stepping: the register-resident kernel for
                           a lone floating body with at most 8 contact
                           candidates, the runtime-topology one otherwise     */
@@ -175,7 +178,7 @@ typedef struct gp_batch_opts {
   int32_t steps_per_launch;  /* steps fused in one launch by every kernel
                                 (0 = 100)                                     */
   int32_t block_size;        /* threads per workgroup, 64/128/256 (0 = 256;
-                                grouped launches 128; the single-body
+                                grouped launches 128; trees 64; the single-body
                                 velocity-stepping kernel 64, or 16 at one
                                 lane per body)                                */
   int32_t lanes_per_mech;    /* FAST free bodies with contacts: lanes sharing

@@ -11,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n", [1, 63, 64, 65, 257])
 def test_device_arrays_match_the_host_calls(gp, n):
-    import torch
+    import ctypes as C
+    from test_gpu_rollouts import _hip
     from gorilla_physics_amd import abi, batch, builders, workloads
     from gorilla_physics_amd.mechanism import Isometry3, ModelDesc, SpatialInertia, body_desc
     box = SpatialInertia.cuboid_at([0, 0, 0], 1.0, 0.1, 0.1, 0.1, "b")
@@ -27,17 +28,36 @@ def test_device_arrays_match_the_host_calls(gp, n):
     q, v, tau = rng.normal(size=b.nq_total), rng.normal(size=b.nv_total), rng.normal(size=b.nv_total)
     print(f"case transfers: {b.n_instances} instances, {b.n_buckets} buckets", flush=True)
 
-    def dev(x):
-        return torch.from_numpy(x).cuda()
-    dq, dv, dt = dev(q), dev(v), dev(tau)
-    b.set_state_dev(dq.data_ptr(), dv.data_ptr())
+    hip, bufs = _hip(), []
+
+    def dev(x):  # a device copy of x
+        p = C.c_void_p()
+        assert hip.hipMalloc(C.byref(p), x.nbytes) == 0
+        bufs.append(p)
+        assert hip.hipMemcpy(p, x.ctypes.data, x.nbytes, 1) == 0
+        return p.value
+
+    def host(p, like):
+        out = np.empty_like(like)
+        assert hip.hipMemcpy(out.ctypes.data, p, out.nbytes, 2) == 0
+        return out
+    try:
+        _check(b, descs, q, v, tau, dev, host, abi)
+    finally:
+        for p in bufs:
+            hip.hipFree(p)
+
+
+def _check(b, descs, q, v, tau, dev, host, abi):
+    dt = dev(tau)
+    b.set_state_dev(dev(q), dev(v))
     b.sync()
     hq, hv = b.get_state()
     assert np.array_equal(hq, q) and np.array_equal(hv, v)
-    oq, ov, oa = torch.zeros_like(dq), torch.zeros_like(dv), torch.zeros_like(dv)
-    b.get_state_dev(oq.data_ptr(), ov.data_ptr())
+    oq, ov, oa = dev(np.zeros_like(q)), dev(np.zeros_like(v)), dev(np.zeros_like(v))
+    b.get_state_dev(oq, ov)
     b.sync()
-    assert np.array_equal(oq.cpu().numpy(), q) and np.array_equal(ov.cpu().numpy(), v)
+    assert np.array_equal(host(oq, q), q) and np.array_equal(host(ov, v), v)
     # torques set either way give the same step
     q[:], v[:] = 0.0, 0.1 * v
     at = 0
@@ -46,13 +66,13 @@ def test_device_arrays_match_the_host_calls(gp, n):
             q[at + 3] = 1.0
         at += descs[i % len(descs)].nq
     out = []
-    for set_tau in (lambda: b.set_tau(tau), lambda: b.set_tau_dev(dt.data_ptr())):
+    for set_tau in (lambda: b.set_tau(tau), lambda: b.set_tau_dev(dt)):
         b.set_tau(None)
         b.set_state(q, v)
         set_tau()
         b.step(1e-4)
-        b.get_vdot_dev(oa.data_ptr())
+        b.get_vdot_dev(oa)
         b.sync()
-        assert np.array_equal(oa.cpu().numpy(), b.get_vdot())
-        out.append(oa.cpu().numpy())
+        assert np.array_equal(host(oa, v), b.get_vdot())
+        out.append(host(oa, v))
     assert np.array_equal(out[0], out[1]) and np.isfinite(out[0]).all()
