@@ -359,11 +359,10 @@ int model_create(const gp_model_desc* d, gp_model** out) {
 Bucket::~Bucket() { release(); }
 
 void Bucket::release() {
-  void* ptrs[] = {d_arena, d_scratch, d_active, d_flat_off};
+  void* ptrs[] = {d_arena, d_scratch, d_active};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   d_arena = nullptr;
-  d_flat_off = nullptr;
   d_sstart = nullptr;
   d_depth = d_child_start = d_child = nullptr;
   d_sp = d_ss = nullptr;
@@ -896,36 +895,51 @@ int gp_batch_create(gp_model* const* models, const int64_t* counts, int32_t n_mo
       bt->qoff[i + 1] = bt->qoff[i] + b.nq;
       bt->voff[i + 1] = bt->voff[i] + b.nv;
     }
-    // each lane's offsets into the flattened arrays, for the device-array calls
-    for (Bucket& b : bt->buckets) {
-      std::vector<int64_t> off(2 * (size_t)b.B);
-      for (int l = 0; l < b.B; ++l) {
-        off[l] = bt->qoff[b.inst[l]];
-        off[b.B + l] = bt->voff[b.inst[l]];
-      }
-      HIP_TRY(hipMalloc((void**)&b.d_flat_off, off.size() * sizeof(int64_t)));
-      HIP_TRY(hipMemcpy(b.d_flat_off, off.data(), off.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    // The transfers' block, one allocation and one copy: each lane's offsets into
+    // the flattened arrays (q, then v, bucket after bucket), the tables (state,
+    // torques, accelerations, gp_dynamics' torques), and a flat staging array
+    // (one q and one v) for the host calls, which do without it if it does not fit.
+    const size_t off_bytes = 2 * (size_t)inst * sizeof(int64_t);
+    const size_t table_bytes = 5 * bt->buckets.size() * sizeof(XferEntry);
+    const size_t head = (off_bytes + table_bytes + 255) / 256 * 256;
+    const size_t staging = (size_t)(bt->qoff.back() + bt->voff.back()) * sizeof(double);
+    const bool fits = hipMalloc(&bt->d_block, head + staging) == hipSuccess;
+    if (!fits) {
+      (void)hipGetLastError();
+      bt->d_block = nullptr;
+      HIP_TRY(hipMalloc(&bt->d_block, head));
     }
-    // and the tables of those calls (state, torques, accelerations)
-    std::vector<XferEntry> xt;
-    for (int which = 0; which < 3; ++which) {
+    char* block = (char*)bt->d_block;
+    bt->d_flat = fits && staging ? (double*)(block + head) : nullptr;
+    bt->d_xfer = (XferEntry*)(block + off_bytes);
+    std::vector<char> h(off_bytes + table_bytes, 0);
+    int64_t* off = (int64_t*)h.data();
+    XferEntry* table = (XferEntry*)(h.data() + off_bytes);
+    int entries = 0;
+    for (int which = 0; which < 4; ++which) {
       gp_batch::Xfer& x = bt->xfer[which];
-      x.at = (int)xt.size();
-      auto add = [&](const Bucket& b, double* soa, int rows, bool second) {
-        if (rows == 0) return;
-        xt.push_back(XferEntry{soa, b.d_flat_off + (second ? b.B : 0), b.Bp, b.B, rows, second ? 1 : 0, x.blocks});
-        x.blocks += (unsigned)((b.B + 63) / 64);
-      };
+      x.at = entries;
+      size_t at = 0;  // the bucket's first offset
       for (const Bucket& b : bt->buckets) {
-        if (which == 0) add(b, b.d_q, b.nq, false);
-        add(b, which == 0 ? b.d_v : which == 1 ? b.d_tau : b.d_vdot, b.nv, true);
+        auto add = [&](double* soa, int rows, bool second) {
+          if (rows == 0) return;
+          table[entries++] = XferEntry{soa, (const int64_t*)block + at + (second ? b.B : 0), b.Bp, b.B, rows,
+                                       second ? 1 : 0, x.blocks};
+          x.blocks += (unsigned)((b.B + 63) / 64);
+        };
+        if (which == 0) {
+          for (int l = 0; l < b.B; ++l) {
+            off[at + l] = bt->qoff[b.inst[l]];
+            off[at + b.B + l] = bt->voff[b.inst[l]];
+          }
+          add(b.d_q, b.nq, false);
+        }
+        add(which == 0 ? b.d_v : which == 1 ? b.d_tau : which == 2 ? b.d_vdot : b.d_tau_tmp, b.nv, true);
+        at += 2 * (size_t)b.B;
       }
-      x.n = (int)xt.size() - x.at;
+      x.n = entries - x.at;
     }
-    if (!xt.empty()) {
-      HIP_TRY(hipMalloc((void**)&bt->d_xfer, xt.size() * sizeof(XferEntry)));
-      HIP_TRY(hipMemcpy(bt->d_xfer, xt.data(), xt.size() * sizeof(XferEntry), hipMemcpyHostToDevice));
-    }
+    HIP_TRY(hipMemcpy(block, h.data(), h.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipStreamCreate(&bt->stream));
     HIP_TRY(hipEventCreate(&bt->ev0));
     HIP_TRY(hipEventCreate(&bt->ev1));
@@ -982,9 +996,61 @@ int gp_batch_get_opts(const gp_batch* bt, gp_batch_opts* o) {
   return GP_OK;
 }
 
-// host flattened (instance-major) <-> bucket SoA
+static int transfer_by_bucket(gp_batch* bt, const double* hq, const double* hv, double* oq, double* ov, bool to_dev,
+                              int which);
+
+// host flattened (instance-major) <-> bucket SoA: one copy between the host
+// and the flat staging array and one transposition launch for every bucket.
+// Both run on the null stream, which waits for (and holds back) every
+// blocking stream, as plain copies do; the call returns when they are done.
+// A batch of one bucket that sets few values copies its rows straight in
+// (transfer_by_bucket): one copy an array and no launch to wait for. By bucket
+// against staged, 7-joint arms: set_tau of 256 16 / 33 us, of 4,096 28 / 31,
+// of 65,536 310 / 143; set_state of 16 34 / 31, of 256 42 / 38, of 65,536
+// 1,462 / 277; get_state of 1 31 / 18, of 65,536 946 / 502.
 static int transfer(gp_batch* bt, const double* hq, const double* hv, double* oq, double* ov, bool to_dev,
-                     int which /*0 state, 1 tau, 2 vdot, 3 tau_tmp*/) {
+                    int which /*0 state, 1 tau, 2 vdot, 3 tau_tmp*/) {
+  double* flat = bt->d_flat;
+  const size_t values = (size_t)(which == 0 ? bt->qoff.back() + bt->voff.back() : bt->voff.back());
+  const bool few = to_dev && bt->buckets.size() == 1 && values <= (which == 0 ? 256u : 32768u);
+  if (!flat || few) return transfer_by_bucket(bt, hq, hv, oq, ov, to_dev, which);
+  const size_t nq = which == 0 ? (size_t)bt->qoff.back() : 0, nv = (size_t)bt->voff.back();
+  const gp_batch::Xfer& x = bt->xfer[which];
+  // small ones cross in one copy, through a host buffer that holds q and v together
+  const bool small = nq > 0 && nv > 0 && (nq + nv) * sizeof(double) <= ((size_t)1 << 20);
+  std::vector<double> both(small ? nq + nv : 0);
+  auto launch = [&]() { return launch_flat_xfer(bt->d_xfer + x.at, x.n, x.blocks, flat, flat + nq, to_dev, nullptr); };
+  if (to_dev) {
+    if (!hv) {
+      std::vector<double> zero(nv, 0.0);
+      HIP_TRY(hipMemcpy(flat, zero.data(), nv * sizeof(double), hipMemcpyHostToDevice));
+    } else if (small) {
+      std::copy(hq, hq + nq, both.begin());
+      std::copy(hv, hv + nv, both.begin() + nq);
+      HIP_TRY(hipMemcpy(flat, both.data(), both.size() * sizeof(double), hipMemcpyHostToDevice));
+    } else {
+      if (nq) HIP_TRY(hipMemcpy(flat, hq, nq * sizeof(double), hipMemcpyHostToDevice));
+      if (nv) HIP_TRY(hipMemcpy(flat + nq, hv, nv * sizeof(double), hipMemcpyHostToDevice));
+    }
+  }
+  const int e = launch();
+  if (e) return fail(GP_ERR_DEVICE, "transposition launch: %s", hipGetErrorString((hipError_t)e));
+  if (to_dev) {
+    HIP_TRY(hipStreamSynchronize(nullptr));
+  } else if (small) {
+    HIP_TRY(hipMemcpy(both.data(), flat, both.size() * sizeof(double), hipMemcpyDeviceToHost));
+    std::copy(both.begin(), both.begin() + nq, oq);
+    std::copy(both.begin() + nq, both.end(), ov);
+  } else {
+    if (nq) HIP_TRY(hipMemcpy(oq, flat, nq * sizeof(double), hipMemcpyDeviceToHost));
+    if (nv) HIP_TRY(hipMemcpy(ov, flat + nq, nv * sizeof(double), hipMemcpyDeviceToHost));
+  }
+  return GP_OK;
+}
+
+// The same bucket by bucket, transposed on the host.
+static int transfer_by_bucket(gp_batch* bt, const double* hq, const double* hv, double* oq, double* ov, bool to_dev,
+                              int which) {
   HIP_TRY(hipStreamSynchronize(bt->stream));
   for (Bucket& b : bt->buckets) {
     const size_t Bp = b.Bp;

@@ -63,7 +63,6 @@ struct Bucket {
   size_t scratch_doubles = 0;
   void* d_arena = nullptr;  // one allocation holding every array above except scratch and active
   size_t arena_bytes = 0;
-  int64_t* d_flat_off = nullptr;  // [2][B]: each lane's q and v offsets in the flattened arrays
   Bucket() = default;
   Bucket(const Bucket&) = delete;
   Bucket& operator=(const Bucket&) = delete;
@@ -87,11 +86,9 @@ struct Bucket {
       d_rounds = o.d_rounds;
       o.d_rounds = nullptr;
       d_active = o.d_active; d_scratch = o.d_scratch; d_arena = o.d_arena; arena_bytes = o.arena_bytes;
-      d_flat_off = o.d_flat_off;
       d_depth = o.d_depth; d_child_start = o.d_child_start; d_child = o.d_child; max_depth = o.max_depth;
       o.d_depth = o.d_child_start = o.d_child = nullptr;
       o.d_arena = nullptr;
-      o.d_flat_off = nullptr;
       o.d_parent = o.d_qoff = o.d_voff = o.d_cstart = o.d_kind = o.d_fault = o.d_active = nullptr;
       o.d_bp = o.d_cp = o.d_hp = o.d_q = o.d_v = o.d_tau = o.d_tau_tmp = o.d_vdot = o.d_scratch = nullptr;
       o.d_bpf = o.d_cpf = o.d_hpf = nullptr;
@@ -139,11 +136,13 @@ struct gp_batch {
   bool group_trees = false;  // every bucket of the group is a tree (launch_grouped_trees)
   int group_lds = 0;         // its LDS bytes per wave
   // device tables of the transfers between flat device arrays and the buckets:
-  // state (q and v), torques, accelerations, each one launch
+  // state (q and v), torques, accelerations, gp_dynamics' torques, each one launch
   struct Xfer { int at = 0, n = 0; unsigned blocks = 0; };
   gp::XferEntry* d_xfer = nullptr;
-  Xfer xfer[3];
+  Xfer xfer[4];
+  double* d_flat = nullptr;  // flat staging array of the host transfers, or null
+  void* d_block = nullptr;   // the allocation that holds these and the lanes' offsets
   ~gp_batch() {
-    if (d_xfer) (void)hipFree(d_xfer);
+    if (d_block) (void)hipFree(d_block);
   }
 };

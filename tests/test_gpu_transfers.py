@@ -76,3 +76,27 @@ def _check(b, descs, q, v, tau, dev, host, abi):
         assert np.array_equal(host(oa, v), b.get_vdot())
         out.append(host(oa, v))
     assert np.array_equal(out[0], out[1]) and np.isfinite(out[0]).all()
+
+
+@pytest.mark.parametrize("n", [63, 64, 65, 16384, 16385, 40000])
+def test_host_arrays_of_one_bucket(gp, n):
+    """Host calls on a batch of one bucket, around the sizes at which rows are
+    copied straight in (256 state values, 32,768 torques) or staged, and a
+    read-back that crosses in one copy or in two (1 MiB): values come back bit
+    for bit, also when only q or v changes, and torques act as set."""
+    from gorilla_physics_amd import batch, workloads
+    b = batch.Batch([batch.Model(workloads.acrobot_desc())], [n])
+    rng = np.random.default_rng(n)
+    q, v = rng.normal(size=2 * n), rng.normal(size=2 * n)
+    for _ in range(2):
+        b.set_state(q, v)
+        hq, hv = b.get_state()
+        assert np.array_equal(hq, q) and np.array_equal(hv, v)
+        v = rng.normal(size=2 * n)
+    b.set_state(q, 0 * v)
+    free, tau = b.dynamics(), rng.normal(size=2 * n)
+    b.set_tau(tau)
+    held = b.dynamics()
+    assert np.array_equal(held, b.dynamics(tau)) and (held != free).any()
+    b.set_tau(None)
+    assert np.array_equal(b.dynamics(), free)
