@@ -124,13 +124,16 @@ class Batch:
     def mass_matrices(self):
         """gp_mass_matrix: M(q) of every instance (a list of nv_i x nv_i arrays)."""
         _, vo = self.offsets()
-        sizes = [int(n) for n in np.diff(vo)]
-        out = np.empty(max(1, sum(n * n for n in sizes)))
+        sizes = np.diff(vo)
+        out = np.empty(max(1, int((sizes * sizes).sum())))
         abi.check(self.lib.gp_mass_matrix(self.handle, _dp(out)), self.lib)
+        # runs of instances of one size are split at once: each matrix is a view
         res, o = [], 0
-        for n in sizes:
-            res.append(out[o:o + n * n].reshape(n, n).copy())
-            o += n * n
+        ends = np.append(np.flatnonzero(np.diff(sizes)) + 1, sizes.size)
+        for first, end in zip(np.append(0, ends[:-1]), ends):
+            k, n = int(end - first), int(sizes[first])
+            res.extend(out[o:o + k * n * n].reshape(k, n, n))
+            o += k * n * n
         return res
 
     def dynamics_bias(self):

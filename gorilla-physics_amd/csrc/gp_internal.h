@@ -139,6 +139,17 @@ struct BucketArgs {
   double* scratch;     // plain kernel: [NPF][nb][Bp] + RK stages
 };
 
+// One bucket of a query over every bucket of a batch (the joint-space terms and
+// dynamics by the tree kernel's one body per lane): its lanes' offsets into
+// the flat v and mass-matrix arrays, its first workgroup (one wave each).
+struct QueryEntry {
+  BucketArgs a;
+  const double* tau_tmp;  // gp_dynamics' torques
+  const int64_t* voff;
+  const int64_t* moff;
+  unsigned first;
+};
+
 // All buckets of a batch in one launch (fast topologies only): bucket b owns
 // workgroups [block_start[b], block_start[b + 1]).
 constexpr int kMaxGroup = 32;
@@ -196,6 +207,13 @@ size_t plain_scratch_doubles(int nb, int nq, int nv, int Bp);
 // velocity stepping (ccd = 1: with continuous collision detection), FP64, one
 // step per launch; scratch as vs_layout
 int launch_vs_step(const BucketArgs& a, double dt, int ccd, int n_steps, void* stream);
+// Queries over a table of buckets that the tree kernel takes, lds = the
+// largest wave's bytes (query_lds_per_wave). Dynamics: vdot rows, with the held
+// torques or tau_tmp. Terms: M (instance-major blocks) or, where M is null,
+// c - tau_c (the v flattening).
+int launch_tree_dynamics(const QueryEntry* d_table, int n, unsigned blocks, int lds, int held, void* stream);
+int launch_tree_terms(const QueryEntry* d_table, int n, unsigned blocks, int lds, double* M, double* c, void* stream);
+int query_lds_per_wave(int nb, int floating);
 // mass matrix and bias c(q, v) - tau_c per lane: out is [nv * nv + nv][Bp]
 // (M row-major, then c); needs the bucket's plain scratch
 int launch_terms(const BucketArgs& a, double* out, void* stream);

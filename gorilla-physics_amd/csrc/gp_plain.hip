@@ -80,6 +80,22 @@ int launch_grouped_trees(const GroupTable* d_table, int n_blocks, int lds_per_wa
   return (int)hipGetLastError();
 }
 
+// dynamics_continuous of every bucket in the table: vdot at the current state,
+// with the held torques or gp_dynamics' own. One wave per workgroup.
+__global__ void __launch_bounds__(64, 2) tree_dynamics_kernel(const QueryEntry* __restrict__ t, int n, int held) {
+  const int e = query_entry(t, n, blockIdx.x);
+  BucketArgs a = t[e].a;
+  if (!held) a.tau = t[e].tau_tmp;
+  wave_tree_body<double, true>(a, (int)(blockIdx.x - t[e].first) * 64 + (int)threadIdx.x, 0.0, 1);
+}
+
+int launch_tree_dynamics(const QueryEntry* d_table, int n, unsigned blocks, int lds, int held, void* stream) {
+  if (n == 0 || blocks == 0) return 0;
+  hipLaunchKernelGGL(tree_dynamics_kernel, dim3(blocks), dim3(64), (unsigned)lds, (hipStream_t)stream, d_table, n,
+                     held);
+  return (int)hipGetLastError();
+}
+
 bool aux_tree_ok(int nb, const int* parent) { return tree_topology_ok(nb, parent); }
 int tree_lds_per_wave(int nb, int floating) { return tree_wave_bytes(nb, floating); }
 

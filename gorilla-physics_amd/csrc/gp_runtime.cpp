@@ -1343,11 +1343,98 @@ int gp_batch_get_vdot(gp_batch* bt, double* vdot) {
   return transfer(bt, nullptr, nullptr, nullptr, vdot, false, 2);
 }
 
+// The queries' table over the buckets that the tree kernel takes (no spring
+// contacts, at most 8 children a body) and the list of the others.
+static int ensure_query(gp_batch* bt) {
+  if (bt->query_built) return GP_OK;
+  bt->moff.assign(bt->n_inst + 1, 0);
+  for (int64_t i = 0; i < bt->n_inst; ++i) {
+    const int64_t nv = bt->voff[i + 1] - bt->voff[i];
+    bt->moff[i + 1] = bt->moff[i] + nv * nv;
+  }
+  std::vector<QueryEntry> table;
+  std::vector<int64_t> moff;  // by entry and lane
+  std::vector<int> other;
+  unsigned blocks = 0;
+  int lds = 0;
+  size_t at = 0;
+  for (size_t k = 0; k < bt->buckets.size(); ++k) {
+    const Bucket& b = bt->buckets[k];
+    if (b.nsp == 0 && aux_tree_ok(b.nb, b.parent.data())) {
+      QueryEntry e{};
+      e.a = bucket_args(b, b.nb, nullptr);
+      e.tau_tmp = b.d_tau_tmp;
+      e.voff = (const int64_t*)bt->d_block + at + b.B;
+      e.first = blocks;
+      blocks += (unsigned)(fast_threads(TOPO_TREE, b.B, b.nb) / 64);
+      lds = std::max(lds, query_lds_per_wave(b.nb, b.nq - b.nv));
+      for (int l = 0; l < b.B; ++l) moff.push_back(bt->moff[b.inst[l]]);
+      table.push_back(e);
+    } else {
+      other.push_back((int)k);
+    }
+    at += 2 * (size_t)b.B;
+  }
+  if (!table.empty()) {
+    const size_t tb = table.size() * sizeof(QueryEntry);
+    void* d = nullptr;
+    hipError_t e = hipMalloc(&d, tb + moff.size() * sizeof(int64_t));
+    if (e != hipSuccess) return fail(GP_ERR_NOMEM, "hipMalloc(query table): %s", hipGetErrorString(e));
+    const int64_t* dm = (const int64_t*)((char*)d + tb);
+    size_t first = 0;
+    for (QueryEntry& x : table) {
+      x.moff = dm + first;
+      first += (size_t)x.a.B;
+    }
+    e = hipMemcpy(d, table.data(), tb, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy((void*)dm, moff.data(), moff.size() * sizeof(int64_t), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+      (void)hipFree(d);
+      return fail(GP_ERR_DEVICE, "query table: %s", hipGetErrorString(e));
+    }
+    bt->d_query = (QueryEntry*)d;
+  }
+  bt->query_n = (int)table.size();
+  bt->query_blocks = blocks;
+  bt->query_lds = lds;
+  bt->query_other = std::move(other);
+  bt->query_built = true;
+  return GP_OK;
+}
+
+// Buckets that a query visits one by one with the one-instance-per-lane
+// kernels: all of them with GP_KERNEL_PLAIN, else those that the tree kernel
+// does not take. One launch over all the others with one body per lane was
+// faster at every size tried (us a call, host arrays, one instance per lane
+// against one body per lane): M of one quadruped 174 / 26, of 8,192 15,919 /
+// 756; c of 8,192 1,310 / 79; vdot of one 12-joint arm 125 / 36, of 65,536
+// 650 / 597.
+static int query_plan(gp_batch* bt, bool* tree, std::vector<int>* rest) {
+  *tree = bt->opts.kernel != GP_KERNEL_PLAIN;
+  if (!*tree) {
+    for (size_t k = 0; k < bt->buckets.size(); ++k) rest->push_back((int)k);
+    return GP_OK;
+  }
+  int st = ensure_query(bt);
+  if (st) return st;
+  *rest = bt->query_other;
+  return GP_OK;
+}
+
 int gp_dynamics(gp_batch* bt, const double* tau, double* vdot) {
   if (!bt || !vdot) return fail(GP_ERR_INVALID, "null argument");
   int st;
   if (tau && (st = transfer(bt, nullptr, tau, nullptr, nullptr, true, 3))) return st;
-  for (Bucket& b : bt->buckets) {
+  bool tree = false;
+  std::vector<int> rest;
+  if ((st = query_plan(bt, &tree, &rest))) return st;
+  if (tree) {
+    // on the null stream, which waits for the batch's
+    int e = launch_tree_dynamics(bt->d_query, bt->query_n, bt->query_blocks, bt->query_lds, tau ? 0 : 1, nullptr);
+    if (e) return fail(GP_ERR_DEVICE, "dynamics launch: %s", hipGetErrorString((hipError_t)e));
+  }
+  for (int k : rest) {
+    Bucket& b = bt->buckets[k];
     if ((st = bucket_ensure_scratch(b))) return st;
     BucketArgs a = bucket_args(b, 1, tau ? b.d_tau_tmp : nullptr);
     int e = launch_plain_step(a, 0.0, GP_SEMI_IMPLICIT_EULER, 1, 1, bt->stream);
@@ -1356,20 +1443,52 @@ int gp_dynamics(gp_batch* bt, const double* tau, double* vdot) {
   return transfer(bt, nullptr, nullptr, nullptr, vdot, false, 2);
 }
 
-// M (instance-major, each nv_i x nv_i row-major) and / or c - tau_c (the v
+// M (instance-major, each nv_i x nv_i row-major) or c - tau_c (the v
 // flattening) of every instance at the batch's state
 static int joint_space_terms(gp_batch* bt, double* Mh, double* ch) {
+  bool tree = false;
+  std::vector<int> rest;
+  int st = query_plan(bt, &tree, &rest);
+  if (st) return st;
+  HIP_TRY(hipStreamSynchronize(bt->stream));
+  if (tree && bt->query_n > 0) {
+    const size_t n = (size_t)(Mh ? bt->moff.back() : bt->voff.back());
+    if (n > 0) {
+      // up to 64 MiB of results stay allocated with the batch
+      constexpr size_t kTermsKept = ((size_t)64 << 20) / sizeof(double);
+      double* d = bt->d_terms;
+      if (n > bt->terms_cap) {
+        if (n <= kTermsKept && bt->d_terms) {
+          (void)hipFree(bt->d_terms);
+          bt->d_terms = nullptr;
+          bt->terms_cap = 0;
+        }
+        hipError_t e = hipMalloc((void**)&d, n * sizeof(double));
+        if (e != hipSuccess) return fail(GP_ERR_NOMEM, "hipMalloc(terms): %s", hipGetErrorString(e));
+        if (n <= kTermsKept) {
+          bt->d_terms = d;
+          bt->terms_cap = n;
+        }
+      }
+      int le = launch_tree_terms(bt->d_query, bt->query_n, bt->query_blocks, bt->query_lds, Mh ? d : nullptr,
+                                 Mh ? nullptr : d, nullptr);
+      // the other buckets' parts are filled in below
+      if (!le) le = (int)hipMemcpy(Mh ? Mh : ch, d, n * sizeof(double), hipMemcpyDeviceToHost);
+      if (d != bt->d_terms) (void)hipFree(d);
+      if (le) return fail(GP_ERR_DEVICE, "joint-space terms: %s", hipGetErrorString((hipError_t)le));
+    }
+  }
+  if (rest.empty()) return GP_OK;
   std::vector<int64_t> moff(bt->n_inst + 1, 0);
   for (int64_t i = 0; i < bt->n_inst; ++i) {
     const int64_t nv = bt->voff[i + 1] - bt->voff[i];
     moff[i + 1] = moff[i] + nv * nv;
   }
-  HIP_TRY(hipStreamSynchronize(bt->stream));
-  for (Bucket& b : bt->buckets) {
+  for (int bk : rest) {
+    Bucket& b = bt->buckets[bk];
     const size_t rows = (size_t)b.nv * b.nv + b.nv;
     if (b.nv == 0 || b.B == 0) continue;
-    int st = bucket_ensure_scratch(b);
-    if (st) return st;
+    if ((st = bucket_ensure_scratch(b))) return st;
     double* d = nullptr;
     hipError_t e = hipMalloc((void**)&d, rows * b.Bp * sizeof(double));
     if (e != hipSuccess) return fail(GP_ERR_NOMEM, "hipMalloc(terms): %s", hipGetErrorString(e));

@@ -142,7 +142,19 @@ struct gp_batch {
   Xfer xfer[4];
   double* d_flat = nullptr;  // flat staging array of the host transfers, or null
   void* d_block = nullptr;   // the allocation that holds these and the lanes' offsets
+  // The queries' table (gp_dynamics, gp_mass_matrix, gp_dynamics_bias), built
+  // on first use: the buckets that the tree kernel takes, and the others' indices
+  bool query_built = false;
+  gp::QueryEntry* d_query = nullptr;
+  int query_n = 0, query_lds = 0;
+  unsigned query_blocks = 0;
+  std::vector<int> query_other;
+  std::vector<int64_t> moff;  // each instance's offset in the mass matrices (n + 1)
+  double* d_terms = nullptr;  // their results, kept while small (kTermsKept)
+  size_t terms_cap = 0;
   ~gp_batch() {
+    if (d_terms) (void)hipFree(d_terms);
+    if (d_query) (void)hipFree(d_query);
     if (d_block) (void)hipFree(d_block);
   }
 };

@@ -130,7 +130,46 @@ __device__ __forceinline__ void ldl6_solve(const double (&L)[21], double (&x)[6]
     for (int k = i + 1; k < 6; ++k) x[i] -= L[k * (k + 1) / 2 + i] * x[k];
 }
 
+// Contact wrench on a body (contact.rs:97-129) in its frame: points [c0, c1)
+// of the bucket against every half-space, the body's world pose (Rw, tw).
 template <class R>
+__device__ __forceinline__ sv<R> tree_contacts(const BucketArgs& a, int inst, int c0, int c1, const m3<double>& Rw,
+                                               const v3<double>& tw, const sv<R>& vel) {
+  const Soa<double> cpS(a.cp, NCF * a.nc, a.Bp), hpS(a.hp, NHF * a.nh, a.Bp);
+  const m3<R> RwR = cvt<R>(Rw);
+  sv<R> fe{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
+  for (int h = 0; h < a.nh; ++h) {
+    auto hpar = [&](int fld) { return hpS.ld(fld * a.nh + h, inst); };
+    const v3<double> n{hpar(HF_NORMAL), hpar(HF_NORMAL + 1), hpar(HF_NORMAL + 2)};
+    const v3<double> nb_ = mulT(Rw, n);
+    const double off = dot(tw - v3<double>{hpar(HF_POINT), hpar(HF_POINT + 1), hpar(HF_POINT + 2)}, n);
+    const R alpha = R(hpar(HF_ALPHA)), mu = R(hpar(HF_MU));
+    for (int cc = c0; cc < c1; ++cc) {
+      auto cpar = [&](int fld) { return cpS.ldx(fld * a.nc, inst, cc); };
+      const v3<double> pb{cpar(CF_P), cpar(CF_P + 1), cpar(CF_P + 2)};
+      const double dist = dot(nb_, pb) + off;
+      if (dist <= kInsideMargin) {
+        const v3<R> pbR = cvt<R>(pb);
+        const v3<R> vw = mul(RwR, vel.v + cross(vel.w, pbR));
+        const v3<R> F = contact_force(R(-dist), cvt<R>(n), vw, R(cpar(CF_K)), R(kHalfspaceK), alpha, mu);
+        const v3<R> Fb = mulT(RwR, F);
+        fe.w = fe.w + cross(pbR, Fb);
+        fe.v = fe.v + Fb;
+      }
+    }
+  }
+  return fe;
+}
+
+// The children's lanes of body j, a byte each
+__device__ __forceinline__ unsigned long long tree_children(const BucketArgs& a, int ch0, int nch) {
+  unsigned long long c = 0;
+  for (int k = 0; k < nch; ++k) c |= (unsigned long long)a.child[ch0 + k] << (8 * k);
+  return c;
+}
+
+// DYN: one evaluation at the batch's state instead of steps, leaving only vdot.
+template <class R, bool DYN = false>
 __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, double dt, int n_steps) {
   const int nb = a.nb, Bp = a.Bp;
   const int ipw = 64 / nb;  // instances per wave
@@ -138,7 +177,7 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
   const int inst = (tid >> 6) * ipw + seg;
   if (seg >= ipw || inst >= a.B) return;  // an instance's lanes leave together
   int my_steps = n_steps;
-  if (a.active) {  // serving: the instance's remaining horizon
+  if (!DYN && a.active) {  // serving: the instance's remaining horizon
     const int left = a.active[inst];
     if (left <= 0) return;
     my_steps = min(my_steps, left);
@@ -148,8 +187,7 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
   const int maxd = a.max_depth;
   const int par = a.parent[j], depth = a.depth[j];
   const int ch0 = a.child_start[j], nch = a.child_start[j + 1] - ch0;
-  unsigned long long child = 0;  // the children's lanes, a byte each
-  for (int k = 0; k < nch; ++k) child |= (unsigned long long)a.child[ch0 + k] << (8 * k);
+  const unsigned long long child = tree_children(a, ch0, nch);
   const int qo = a.qoff[j], vo = a.voff[j];
   const Soa<int> kindS(a.kind, nb, Bp);
   const int kind = kindS.ldx(0, inst, j);
@@ -175,7 +213,6 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
   const double sk = kind == K_PRI ? pd(BF_SK) : 0.0;
   const double sl = kind == K_PRI ? pd(BF_SL) : 0.0;
   const Soa<double> qS(a.q, a.nq, Bp), vS(a.v, a.nv, Bp), tauS(a.tau, a.nv, Bp), vdotS(a.vdot, a.nv, Bp);
-  const Soa<double> cpS(a.cp, NCF * a.nc, Bp), hpS(a.hp, NHF * a.nh, Bp);
   double q = 0.0, v = 0.0, tau = 0.0, vd = 0.0;  // of a one-DOF joint
   if (one) {
     q = qS.ldx(0, inst, qo);
@@ -258,31 +295,7 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
       const v3<R> g = cross(vel.w, vel.v), hw = mul(J, vel.w), wc = cross(vel.w, mc);
       pA = sv<R>{cross(vel.w, hw) + cross(mc, g), mass * g + cross(vel.w, wc)};
     }
-    if (contacts && c0 < c1) {
-      const m3<R> RwR = cvt<R>(Rw);
-      sv<R> fe{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
-      for (int h = 0; h < a.nh; ++h) {
-        auto hpar = [&](int fld) { return hpS.ld(fld * a.nh + h, inst); };
-        const v3<double> n{hpar(HF_NORMAL), hpar(HF_NORMAL + 1), hpar(HF_NORMAL + 2)};
-        const v3<double> nb_ = mulT(Rw, n);
-        const double off = dot(tw - v3<double>{hpar(HF_POINT), hpar(HF_POINT + 1), hpar(HF_POINT + 2)}, n);
-        const R alpha = R(hpar(HF_ALPHA)), mu = R(hpar(HF_MU));
-        for (int cc = c0; cc < c1; ++cc) {
-          auto cpar = [&](int fld) { return cpS.ldx(fld * a.nc, inst, cc); };
-          const v3<double> pb{cpar(CF_P), cpar(CF_P + 1), cpar(CF_P + 2)};
-          const double dist = dot(nb_, pb) + off;
-          if (dist <= kInsideMargin) {
-            const v3<R> pbR = cvt<R>(pb);
-            const v3<R> vw = mul(RwR, vel.v + cross(vel.w, pbR));
-            const v3<R> F = contact_force(R(-dist), cvt<R>(n), vw, R(cpar(CF_K)), R(kHalfspaceK), alpha, mu);
-            const v3<R> Fb = mulT(RwR, F);
-            fe.w = fe.w + cross(pbR, Fb);
-            fe.v = fe.v + Fb;
-          }
-        }
-      }
-      pA = pA - fe;
-    }
+    if (contacts && c0 < c1) pA = pA - tree_contacts<R>(a, inst, c0, c1, Rw, tw, vel);
     // ---- pass 2, leaves to root by depth: articulated inertias and bias forces
     ai6<R> IA = I;
     sv<R> U{{R(0), R(0), R(0)}, {R(0), R(0), R(0)}};
@@ -359,6 +372,7 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
         if (d < maxd) put_sv(mineR, ap);  // slot (R): acceleration from the start
       }
     }
+    if constexpr (DYN) break;
     // ---- semi-implicit Euler of this lane's joint (integrators.rs:276-319); a
     // non-finite acceleration leaves v non-finite for good
     if (kind == K_FLOAT) {
@@ -379,23 +393,25 @@ __device__ __forceinline__ void wave_tree_body(const BucketArgs& a, int tid, dou
     }
   }
   if (one) {
-    qS.stx(0, inst, qo, q);
-    vS.stx(0, inst, vo, v);
+    if constexpr (!DYN) {
+      qS.stx(0, inst, qo, q);
+      vS.stx(0, inst, vo, v);
+    }
     vdotS.stx(0, inst, vo, vd);
-    ok = ok && isfinite(q) && isfinite(v);
+    ok = ok && isfinite(q) && isfinite(v) && isfinite(vd);
   } else if (kind == K_FLOAT) {
 #pragma unroll
     for (int k = 0; k < 7; ++k) {
       const double x = fl[k];
-      qS.stx(k, inst, qo, x);
+      if constexpr (!DYN) qS.stx(k, inst, qo, x);
       ok = ok && isfinite(x);
     }
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      const double x = fl[7 + k];
-      vS.stx(k, inst, vo, x);
-      vdotS.stx(k, inst, vo, fl[19 + k]);
-      ok = ok && isfinite(x);
+      const double x = fl[7 + k], y = fl[19 + k];
+      if constexpr (!DYN) vS.stx(k, inst, vo, x);
+      vdotS.stx(k, inst, vo, y);
+      ok = ok && isfinite(x) && isfinite(y);
     }
   }
   if (!ok) a.fault[inst] = 1;  // any lane's fault is the instance's
@@ -418,6 +434,16 @@ __global__ void __launch_bounds__(256, 2) grouped_tree_kernel(const GroupTable* 
   wave_tree_body<R>(a, tid, dt, n_steps);
 }
 
+// The table entry that owns workgroup b (uniform), for a query over every bucket.
+__device__ __forceinline__ int query_entry(const QueryEntry* t, int n, unsigned b) {
+  int e = 0;
+  for (int hi = n; hi - e > 1;) {
+    const int mid = (e + hi) / 2;
+    if (t[mid].first <= b) e = mid;
+    else hi = mid;
+  }
+  return e;
+}
 template <class R>
 static int launch_wave_tree(const BucketArgs& a, double dt, int n_steps, int block, hipStream_t s) {
   dim3 blk(block), grid((unsigned)((fast_threads(TOPO_TREE, a.B, a.nb) + block - 1) / block));

@@ -97,3 +97,31 @@ def test_small_trees_in_one_launch_give_the_same_bits(gp):
             ref = got
         assert all(np.array_equal(x, y) for x, y in zip(ref, got)), kw
     b.step(1e-4, n_steps=0)
+
+
+@pytest.mark.parametrize("nb", [1, 2, 9, 21, 22, 33, 64])
+@pytest.mark.parametrize("root", ["floating", "revolute", "two"])
+def test_joint_space_terms_of_packed_trees(gp, oracle, nb, root):
+    """M, c and vdot of every instance by the one-body-per-lane kernels and by
+    the one-instance-per-lane ones (GP_KERNEL_PLAIN), each against the
+    oracle's CRBA, RNEA and LU, e <= 1e-10 (the FP64 bound)."""
+    from gorilla_physics_amd import batch
+    from gpu_helpers import rel_err
+    rng = np.random.default_rng(300 * nb + len(root))
+    d = _tree(rng, nb, root)
+    n = 64 // nb + 1
+    parts = [_state(d, rng) for _ in range(n)]
+    q, v, tau = (np.concatenate([p[k] for p in parts]) for k in range(3))
+    print(f"case terms of small tree: {nb} bodies, root {root}, {n} instances", flush=True)
+    for kernel in (0, 1):
+        b = batch.Batch([batch.Model(d)], [n], kernel=kernel)
+        b.set_state(q, v)
+        b.set_tau(tau)
+        Ms, c, held, given = b.mass_matrices(), b.dynamics_bias(), b.dynamics(), b.dynamics(2.0 * tau)
+        assert len(Ms) == n and not b.faults().any()
+        for i, (qi, vi, ti) in enumerate(parts):
+            Mr, cr = oracle.mass_matrix(d, qi, vi)
+            s = slice(i * d.nv, (i + 1) * d.nv)
+            assert rel_err(Ms[i], Mr) <= TOL and rel_err(c[s], cr) <= TOL and np.array_equal(Ms[i], Ms[i].T)
+            assert rel_err(held[s], oracle.dynamics(d, qi, vi, ti)) <= TOL
+            assert rel_err(given[s], oracle.dynamics(d, qi, vi, 2.0 * ti)) <= TOL
