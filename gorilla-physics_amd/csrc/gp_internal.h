@@ -207,6 +207,10 @@ size_t plain_scratch_doubles(int nb, int nq, int nv, int Bp);
 // velocity stepping (ccd = 1: with continuous collision detection), FP64, one
 // step per launch; scratch as vs_layout
 int launch_vs_step(const BucketArgs& a, double dt, int ccd, int n_steps, void* stream);
+// the same step with one instance per wave, the same bits; vs_wave_ok: whether
+// the bucket's sizes fit and its instances are few enough for it to be faster
+int launch_vs_wave(const BucketArgs& a, double dt, int ccd, int n_steps, void* stream);
+bool vs_wave_ok(int B, int nb, int nq, int nv, int nc, int nh, int ns);
 // Queries over a table of buckets that the tree kernel takes, lds = the
 // largest wave's bytes (query_lds_per_wave). Dynamics: vdot rows, with the held
 // torques or tau_tmp. Terms: M (instance-major blocks) or, where M is null,

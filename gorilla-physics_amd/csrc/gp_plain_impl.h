@@ -27,11 +27,19 @@ struct Strided {  // a[k] of one lane in a [k][Bp] array
   __device__ double& operator[](int k) const { return p[(size_t)k * Bp]; }
 };
 
+// One instance's bodies: its per-body fields are a [NPF][nb] block at sc with
+// `pitch` between values (a lane's column of the bucket's scratch, or a
+// contiguous block of its own).
 struct PlainCtx {
   const BucketArgs& a;
   int lane;
+  double* sc;
+  int pitch;
+  __device__ PlainCtx(const BucketArgs& a_, int lane_) : PlainCtx(a_, lane_, a_.scratch + lane_, a_.Bp) {}
+  __device__ __forceinline__ PlainCtx(const BucketArgs& a_, int lane_, double* sc_, int pitch_)
+      : a(a_), lane(lane_), sc(sc_), pitch(pitch_) {}
   __device__ double bpar(int f, int i) const { return a.bp[((size_t)f * a.nb + i) * a.Bp + lane]; }
-  __device__ double& s(int f, int i) const { return a.scratch[((size_t)f * a.nb + i) * a.Bp + lane]; }
+  __device__ double& s(int f, int i) const { return sc[((size_t)f * a.nb + i) * pitch]; }
   __device__ void st3(int f, int i, v3<double> x) const { s(f, i) = x.x; s(f + 1, i) = x.y; s(f + 2, i) = x.z; }
   __device__ v3<double> ld3(int f, int i) const { return {s(f, i), s(f + 1, i), s(f + 2, i)}; }
   __device__ void stv(int f, int i, const sv<double>& x) const { st3(f, i, x.w); st3(f + 3, i, x.v); }
@@ -69,9 +77,10 @@ struct PlainCtx {
 // registration (a query: a spring registering in this evaluation, or
 // detaching, exerts no force either way). Returns false where a spring
 // contact pulls into its half-space.
-__device__ inline bool plain_kinematics(const BucketArgs& a, int lane, Strided q, Strided v, bool contacts = true,
-                                        bool update_springs = true) {
-  PlainCtx X{a, lane};
+__device__ __forceinline__ bool plain_kinematics_on(const PlainCtx& X, Strided q, Strided v, bool contacts,
+                                                    bool update_springs) {
+  const BucketArgs& a = X.a;
+  const int lane = X.lane;
   const int nb = a.nb, Bp = a.Bp;
   bool ok = true;
   for (int i = 0; i < nb; ++i) {
@@ -189,16 +198,22 @@ __device__ inline bool plain_kinematics(const BucketArgs& a, int lane, Strided q
   return ok;
 }
 
+__device__ inline bool plain_kinematics(const BucketArgs& a, int lane, Strided q, Strided v, bool contacts = true,
+                                        bool update_springs = true) {
+  return plain_kinematics_on(PlainCtx{a, lane}, q, v, contacts, update_springs);
+}
+
 // Articulated-body forward dynamics of one lane; q, v, tau, vdot are the
 // lane's columns of [k][Bp] arrays. contacts = false leaves out the contact
 // and spring-contact forces (the velocity-stepping path). Returns false on a
 // non-positive D.
-__device__ inline bool plain_dynamics(const BucketArgs& a, int lane, Strided q, Strided v, Strided tau, Strided vdot,
-                                      bool contacts = true) {
-  PlainCtx X{a, lane};
+__device__ __forceinline__ bool plain_dynamics_on(const PlainCtx& X, Strided q, Strided v, Strided tau, Strided vdot,
+                                                  bool contacts) {
+  const BucketArgs& a = X.a;
+  const int lane = X.lane;
   const int nb = a.nb, Bp = a.Bp;
   // ---- pass 1: kinematics, velocities, bias forces, contact forces
-  bool ok = plain_kinematics(a, lane, q, v, contacts);
+  bool ok = plain_kinematics_on(X, q, v, contacts, true);
   // ---- pass 2: articulated inertias and bias forces, leaves to root
   for (int i = nb - 1; i >= 0; --i) {
     const int k = a.kind[i * Bp + lane];
@@ -277,8 +292,13 @@ __device__ inline bool plain_dynamics(const BucketArgs& a, int lane, Strided q, 
   return ok;
 }
 
+__device__ inline bool plain_dynamics(const BucketArgs& a, int lane, Strided q, Strided v, Strided tau, Strided vdot,
+                                      bool contacts = true) {
+  return plain_dynamics_on(PlainCtx{a, lane}, q, v, tau, vdot, contacts);
+}
+
 // q_out = q (+) h v  for every joint of the lane
-__device__ inline void plain_advance(const BucketArgs& a, int lane, Strided q, Strided v, double h, Strided qo) {
+__device__ __forceinline__ void plain_advance(const BucketArgs& a, int lane, Strided q, Strided v, double h, Strided qo) {
   for (int i = 0; i < a.nb; ++i) {
     const int k = a.kind[i * a.Bp + lane];
     const int o = a.qoff[i], w = a.voff[i];
@@ -294,7 +314,7 @@ __device__ inline void plain_advance(const BucketArgs& a, int lane, Strided q, S
   }
 }
 
-__device__ inline bool finite_cols(Strided x, int n) {
+__device__ __forceinline__ bool finite_cols(Strided x, int n) {
   bool ok = true;
   for (int k = 0; k < n; ++k) ok = ok && isfinite(x[k]);
   return ok;

@@ -710,9 +710,10 @@ static int batch_launch_all(gp_batch* bt, double dt, int integrator, int n_steps
       if (st) return st;
       BucketArgs a = bucket_args(b, 1, nullptr);
       if (scratch_override) a.scratch = scratch_override;
+      const bool wave = o.kernel != GP_KERNEL_PLAIN && vs_wave_ok(b.B, b.nb, b.nq, b.nv, b.nc, b.nh, b.ns);
       for (int done = 0; done < n_steps; done += spl) {
         const int n = std::min(spl, n_steps - done);
-        int e = launch_vs_step(a, dt, ccd, n, s);
+        int e = wave ? launch_vs_wave(a, dt, ccd, n, s) : launch_vs_step(a, dt, ccd, n, s);
         if (e) return fail(GP_ERR_DEVICE, "velocity-stepping launch: %s", hipGetErrorString((hipError_t)e));
         ++*launches;
       }

@@ -88,10 +88,12 @@ enum {
                           body per lane, FP64;
                           velocity stepping: the register-resident kernel for
                           a lone floating body with at most 8 contact
-                          candidates, the runtime-topology one otherwise     */
+                          candidates, for others one instance per wave up to
+                          1,024 instances (and 21 candidates), then one per
+                          lane                                               */
   GP_KERNEL_PLAIN = 1, /* runtime-topology FP64 kernel, per-body
                           intermediates in device scratch (also for velocity
-                          stepping)                                          */
+                          stepping, one instance per lane)                   */
   GP_KERNEL_FAST = 2   /* compile-time topology, register resident, several
                           steps per launch                                     */
 };

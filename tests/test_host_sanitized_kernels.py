@@ -354,3 +354,45 @@ def test_chain_frames_match_the_oracle(gp, oracle, host_binary_fast, tmp_path, t
         eq, ev, ea = step_errors(oracle, descs, q, v, tau, q1, v1, a1, 1e-3, integrator)
         print(f"turned chains {turn}, integrator {integrator}: {eq.max():.3g} {ev.max():.3g} {ea.max():.3g}")
         assert max(eq.max(), ev.max(), ea.max()) <= 1e-10
+
+
+@pytest.mark.parametrize("integrator", [3, 4])
+def test_wave_velocity_stepping_gives_the_lane_kernels_bits(gp, host_binary, tmp_path, integrator):
+    """Velocity stepping with one instance per wave (the automatic choice for
+    few instances) against the one-instance-per-lane kernel (GP_KERNEL_PLAIN),
+    under the sanitizers: quadrupeds, arms with a sphere on the last link and
+    a cube that touches two planes (more candidates than the single-body kernel takes), in contact
+    and in flight: the same bits of q, v and vdot and the same rounds."""
+    from gorilla_physics_amd import builders
+    from gorilla_physics_amd.mechanism import ModelDesc, halfspace_desc, contact_desc
+    from gorilla_physics_amd import abi
+    rng = np.random.default_rng(21)
+    plane = gp.HalfSpace.new([0.0, 0.0, 1.0], 0.0)
+    quad, cube = builders.build_quadruped(), builders.build_cube(1.0, 1.0)
+    for st in (quad, cube):
+        st.add_halfspace(plane)
+    cube.add_halfspace(gp.HalfSpace.new([np.sin(0.3), 0.0, np.cos(0.3)], 0.0))
+    arm = _turned_chain(gp, rng, 4, "any", 0, True)
+    ball = abi.gp_sphere_desc()
+    ball.body, ball.enabled, ball.radius = 3, 1, 0.2
+    arm = ModelDesc([arm._bodies[i] for i in range(4)], [contact_desc(2, [0.1, 0.0, 0.2], 50e3)],
+                    [halfspace_desc(plane)], spheres=[ball])
+    descs, q, v = [], [], []
+    for k in range(12):
+        d = (quad, cube, arm)[k % 3]
+        d = d if isinstance(d, ModelDesc) else d.model_desc()
+        qi = rng.normal(0.0, 0.2, d.nq)
+        if d.nq != 4:
+            qi[:7] = [0.0, 0.0, 0.0, 1.0, 0.0, 0.0, rng.uniform(0.95, 1.0) if d.nq > 7 else rng.uniform(0.45, 0.7)]
+        descs.append(d), q.append(qi), v.append(rng.normal(0.0, 0.5, d.nv))
+    q, v = np.concatenate(q), np.concatenate(v)
+    tau = rng.normal(0.0, 0.1, v.size)
+    got = []
+    for kernel in (0, 1):
+        out = tmp_path / f"out{kernel}.bin"
+        _run(host_binary, tmp_path, out=out, kernel=kernel, models=descs, counts=[1] * len(descs), q=q, v=v, tau=tau,
+             dt=1e-2, integrator=integrator, steps=8, spl=3)
+        got.append(_read_out(out, q.size, v.size))
+    assert np.isfinite(got[0][0]).all()
+    for x, y in zip(*got):
+        assert np.array_equal(x, y)
