@@ -224,14 +224,14 @@ int launch_terms(const BucketArgs& a, double* out, void* stream);
 // kinetic and gravitational energy per lane (ke[lane], pe[lane])
 int launch_energy(const BucketArgs& a, double* ke, double* pe, void* stream);
 size_t vs_scratch_doubles(int nb, int nq, int nv, int nc, int nh, int ns, int Bp);
-// velocity stepping of a lone floating body, `lanes` (1 or 8) lanes per
-// instance sharing its `candidates` contact candidates (contact points x
-// half-spaces, plus the sphere's half-spaces), the working set in registers
-// and LDS. hipErrorInvalidValue when the candidates do not fit (more than
-// kVsBodyMaxCandidates). block: lanes per workgroup at 8 lanes per body (64,
-// 128 or 256, the same bits; 0 = kVsBodyBlock: one wave per workgroup, so a
-// SIMD whose wave ends takes the next one without waiting for a workgroup's
-// slowest, 1.8 % faster than 256 on the thrown cubes).
+// velocity stepping of a lone floating body with `candidates` contact
+// candidates (contact points x half-spaces, plus the sphere's half-spaces), the
+// working set in registers and LDS: one lane per instance (lanes = 1), else 4
+// or 8 lanes sharing it. hipErrorInvalidValue when the candidates do not fit
+// (more than kVsBodyMaxCandidates). block: lanes per workgroup otherwise than
+// at one lane (64, 128 or 256, the same bits; 0 = kVsBodyBlock: one wave per
+// workgroup, so that a SIMD whose wave ends takes the next one without waiting
+// for a workgroup's slowest).
 constexpr int kVsBodyMaxCandidates = 8;
 constexpr int kVsBodyBlock = 64;
 int launch_vs_body(const BucketArgs& a, double dt, int ccd, int n_steps, int lanes, int candidates, int block,

@@ -13,22 +13,38 @@
 // predictor-corrector, the Cholesky factor of G + D W^-2 D, the same start,
 // stopping and best-iterate rules), v_next = v_free + Y x, and the same
 // collision loop. What differs is where it runs: L lanes share an instance,
-// each holding the rows of T = 8 / L candidates (R = 3 T rows of the 24-row
-// program; an inactive candidate's rows are identity rows with a zero right-
-// hand side, which leaves the active rows' arithmetic unchanged), every
-// working array of the program in registers except G's rows, which sit in a
-// lane-private LDS row (written once per collision round, read each
-// iteration). The Cholesky factorisation is row-distributed: at column j the
-// lane owning row j broadcasts it, every lane updates its own rows; the
-// triangular solves broadcast each solved entry. Sums over rows of different
-// lanes are xor butterflies (commutative adds: every lane holds the same
-// bits and takes the same branches). At 8 lanes, each collision round puts
-// the touching candidates on an instance's first lanes and the wave skips the
-// program's columns past 3 x its largest touching count; broadcasts and sums
-// are DPP moves; the instance's long-lived state waits in LDS while the
+// each holding the rows of T contacts of the program (R = 3 T rows; a contact
+// that does not touch has identity rows with a zero right-hand side, which
+// leaves the others' arithmetic unchanged), every working array of the program
+// in registers except G's rows, which sit in a lane-private LDS row (written
+// once per collision round, read each iteration). The Cholesky factorisation is
+// row-distributed: at column j the lane owning row j broadcasts it, every lane
+// updates its own rows; the triangular solves broadcast each solved entry. Sums
+// over rows of different lanes are xor butterflies (commutative adds: every
+// lane holds the same bits and takes the same branches). Each collision round
+// puts the touching candidates on an instance's first lanes and the wave skips
+// the program's columns past 3 x its largest touching count; broadcasts and
+// sums are DPP moves; the instance's long-lived state waits in LDS while the
 // interior point runs. M is the body's spatial inertia in its frame (the
 // joint-space mass matrix of a floating joint).
+//
+// Four lanes an instance, two candidates and one contact of a 12-row program
+// each: a box on a plane touches with at most its four lowest corners, and 16
+// instances share a wave's instructions. An instance that comes to more
+// contacts leaves with its state at that step's start and is finished by eight
+// lanes and the 24-row program after the wave's others: the same bits, as the
+// rows that are left out are the identity's. At one lane an instance all rows
+// are its own.
+//
+// What bounds it: instruction issue. A wave runs one instance's serial program
+// for all of its instances and waits in each iteration, and at its end, for the
+// slowest of them; collision rounds differ (mean 1.05 to 2.7, at most 14 a step
+// over 24 steps of thrown cubes). 24 steps of 16,384 thrown cubes: 17.05 ms with
+// every step ended together, 14.26 with one loop over all steps' rounds on 8
+// lanes an instance, 7.42 on 4 lanes (1,024 waves, one a SIMD).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "gp_cone.h"
 #include "gp_device.h"
@@ -45,7 +61,9 @@ namespace gp {
 namespace {
 
 constexpr int kBodyCand = kVsBodyMaxCandidates;  // candidates per instance
-constexpr int kBodyRows = 3 * kBodyCand;  // rows of the padded program
+// contacts that the program of L lanes an instance holds: 4 lanes hold one
+// each (and two candidates), 8 lanes or 1 all eight candidates
+template <int L> constexpr int body_cap() { return L == 4 ? 4 : kBodyCand; }
 // doubles of an instance's parked state: q, v (the step's start), the
 // current q and v, v_free, the world rotation and translation
 constexpr int kStash = 7 + 6 + 7 + 6 + 6 + 9 + 3;
@@ -63,12 +81,16 @@ template <int S> __device__ __forceinline__ double bcast8(double x) {
   if constexpr (S < 4) return dpp64<kDppRowShr4, 0xA>(t, t);
   else return dpp64<kDppRowShl4, 0x5>(t, t);
 }
+// lane S of the quad
+template <int S> __device__ __forceinline__ double bcast4(double x) {
+  return dpp64<S | (S << 2) | (S << 4) | (S << 6), 0xF>(x, x);
+}
 
 template <int L> __device__ __forceinline__ double gsum(double x) {
-  if constexpr (L == 8) {
+  if constexpr (L >= 4) {
     x += xor8<1>(x);
     x += xor8<2>(x);
-    return x + xor8<4>(x);
+    return L == 8 ? x + xor8<4>(x) : x;
   } else {
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) x += __shfl_xor(x, o, 64);
@@ -76,10 +98,10 @@ template <int L> __device__ __forceinline__ double gsum(double x) {
   }
 }
 template <int L> __device__ __forceinline__ double gmax(double x) {
-  if constexpr (L == 8) {
+  if constexpr (L >= 4) {
     x = fmax(x, xor8<1>(x));
     x = fmax(x, xor8<2>(x));
-    return fmax(x, xor8<4>(x));
+    return L == 8 ? fmax(x, xor8<4>(x)) : x;
   } else {
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) x = fmax(x, __shfl_xor(x, o, 64));
@@ -87,10 +109,10 @@ template <int L> __device__ __forceinline__ double gmax(double x) {
   }
 }
 template <int L> __device__ __forceinline__ double gmin(double x) {
-  if constexpr (L == 8) {
+  if constexpr (L >= 4) {
     x = fmin(x, xor8<1>(x));
     x = fmin(x, xor8<2>(x));
-    return fmin(x, xor8<4>(x));
+    return L == 8 ? fmin(x, xor8<4>(x)) : x;
   } else {
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) x = fmin(x, __shfl_xor(x, o, 64));
@@ -112,13 +134,20 @@ template <int L> __device__ __forceinline__ double bc(double x, int src) {
       case 6: return bcast8<6>(x);
       default: return bcast8<7>(x);
     }
+  } else if constexpr (L == 4) {
+    switch (src) {
+      case 0: return bcast4<0>(x);
+      case 1: return bcast4<1>(x);
+      case 2: return bcast4<2>(x);
+      default: return bcast4<3>(x);
+    }
   } else return __shfl(x, src, L);
 }
 // the smallest (t, key) over the lanes, the smaller key on a tie
 template <int L, int O> __device__ __forceinline__ void argmin_step(double& t, int& key) {
   double t2;
   int k2;
-  if constexpr (L == 8) {
+  if constexpr (L >= 4) {
     t2 = xor8<O>(t);
     k2 = xor8<O>(key);
   } else {
@@ -146,12 +175,20 @@ struct Cand {
   double hpt[3], hn[3];
 };
 
-template <int L>
-__device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_steps, double* lds) {
-  constexpr int T = kBodyCand / L, R = 3 * T, m = kBodyRows;
+// RESUME: instances that the 4-lane program left at a step (rounds[] =
+// -(step + 1)) go on from there; the others are done.
+template <int L, bool RESUME>
+__device__ void vs_body(const BucketArgs& a, int inst, int sub, double dt, int ccd, int n_steps, double* lds) {
+  constexpr int CT = kBodyCand / L;                     // candidates of a lane, c = t L + sub
+  constexpr int T = body_cap<L>() / L, R = 3 * T, m = 3 * body_cap<L>();  // the program's contacts and rows
   constexpr int pitch = (R * m) | 1;
-  const int inst = tid / L, sub = tid % L;
   if (inst >= a.B) return;
+  int step = 0;
+  if constexpr (RESUME) {
+    const int left_at = a.rounds[inst];
+    if (left_at >= 0) return;
+    step = -left_at - 1;
+  }
   double* Gs = lds + (size_t)threadIdx.x * pitch;  // this lane's rows of G: Gs[i * m + k]
   const int Bp = a.Bp, nb = a.nb, nc = a.nc, nh = a.nh;
   auto bpar = [&](int f) { return a.bp[(size_t)f * nb * Bp + inst]; };
@@ -160,10 +197,10 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
   const int sl = a.ns > 0 ? a.sphere_of[0] : -1;
   const bool sphere_on = sl >= 0 && a.shp[((size_t)SH_ON * a.ns + sl) * Bp + inst] != 0.0;
   const int np = nc * nh, P = np + (sphere_on ? nh : 0);
-  Cand cd[T];
+  Cand cd[CT];
 #pragma unroll
-  for (int t = 0; t < T; ++t) {
-    const int c = sub * T + t;
+  for (int t = 0; t < CT; ++t) {
+    const int c = t * L + sub;
     Cand& C = cd[t];
     C.kind = c < np ? 0 : (c < P ? 1 : -1);
     C.hh = C.kind == 0 ? c % nh : (C.kind == 1 ? c - np : 0);
@@ -186,8 +223,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
 
   // One pass of this loop is one collision round; an instance goes on to its
   // next step when its own step is done, not when the wave's slowest is (a
-  // round's values depend on the instance's own state only). A cube takes 1 to
-  // 10 rounds a step: 24 steps of 16,384 thrown cubes 17.05 -> 14.26 ms.
+  // round's values depend on the instance's own state only).
   double qc[7], vc[6], vn[6];
 #pragma unroll
   for (int k = 0; k < 7; ++k) qc[k] = q[k];
@@ -196,7 +232,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
   bool ok = true;
   double t_remain = dt;
   int forced_h = -1, rounds = 0, last_rounds = 0;
-  for (int step = 0; step < n_steps;) {
+  while (step < n_steps) {
     ++rounds;
     bool done = false;
     const double h = t_remain;
@@ -229,7 +265,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
 #pragma unroll
       for (int k = 0; k < 6; ++k) vfree[k] = vc[k] + h * acc[k];
     }
-    // This round's candidates, cw: for L = 8 the group's touching ones on
+    // This round's candidates, cw: for L = 8 or 4 the group's touching ones on
     // its first lanes in candidate order, the others after them (cd keeps
     // the candidate order, so the layout depends on this round's contacts
     // only, not on how the steps are split into launches). The program's
@@ -242,19 +278,32 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
     Cand cw[T];
 #pragma unroll
     for (int t = 0; t < T; ++t) cw[t] = cd[t];
-    int mw = kBodyCand;
-    if constexpr (L == 8) {
-      bool touch;
-      {
-        const Cand& C = cd[0];
+    int mw = body_cap<L>();
+    if constexpr (L >= 4) {
+      unsigned gmask = 0;  // the instance's touching candidates
+#pragma unroll
+      for (int t = 0; t < CT; ++t) {
+        const Cand& C = cd[t];
         const v3<double> pw = mul(Rw, v3<double>{C.pb[0], C.pb[1], C.pb[2]}) + tw;
         const v3<double> n{C.hn[0], C.hn[1], C.hn[2]};
         const double dist = dot(pw - v3<double>{C.hpt[0], C.hpt[1], C.hpt[2]}, n);
-        touch = C.kind == 0 ? dist <= kInsideMargin : (C.kind == 1 ? (dist <= C.r || C.hh == forced_h) : false);
+        const bool touch = C.kind == 0 ? dist <= kInsideMargin : (C.kind == 1 ? (dist <= C.r || C.hh == forced_h) : false);
+        const unsigned long long wm = __ballot(touch);
+        gmask |= ((unsigned)(wm >> ((threadIdx.x & 63) / L * L)) & ((1u << L) - 1)) << (t * L);
       }
-      const unsigned long long wm = __ballot(touch);
-      const unsigned gmask = (unsigned)(wm >> (8 * ((threadIdx.x & 63) >> 3))) & 0xFFu;
       const int na = __popc(gmask);
+      if constexpr (L == 4) {
+        if (na > body_cap<L>()) {  // more contacts than fit: the 8-lane program takes over from this step's start
+          if (sub == 0) {
+#pragma unroll
+            for (int k = 0; k < 7; ++k) a.q[(size_t)k * Bp + inst] = q[k];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) a.v[(size_t)k * Bp + inst] = v[k];
+            a.rounds[inst] = -(step + 1);
+          }
+          return;
+        }
+      }
       int src = 0, ca = 0, ci = 0;  // the lane whose candidate this lane takes
 #pragma unroll
       for (int b = 0; b < 8; ++b) {
@@ -267,19 +316,27 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
         }
       }
       Cand& C = cw[0];
-      C.kind = __shfl(C.kind, src, 8);
-      C.hh = __shfl(C.hh, src, 8);
-      C.id = __shfl(C.id, src, 8);
-      C.r = __shfl(C.r, src, 8);
+      auto take = [&](auto field) {
+        auto x = __shfl(field(cd[0]), src % L, L);
+        if constexpr (CT > 1) {
+          const auto y = __shfl(field(cd[CT - 1]), src % L, L);
+          x = src < L ? x : y;
+        }
+        return x;
+      };
+      C.kind = take([](const Cand& c) { return c.kind; });
+      C.hh = take([](const Cand& c) { return c.hh; });
+      C.id = take([](const Cand& c) { return c.id; });
+      C.r = take([](const Cand& c) { return c.r; });
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        C.pb[k] = __shfl(C.pb[k], src, 8);
-        C.hpt[k] = __shfl(C.hpt[k], src, 8);
-        C.hn[k] = __shfl(C.hn[k], src, 8);
+        C.pb[k] = take([&](const Cand& c) { return c.pb[k]; });
+        C.hpt[k] = take([&](const Cand& c) { return c.hpt[k]; });
+        C.hn[k] = take([&](const Cand& c) { return c.hn[k]; });
       }
       mw = 0;
 #pragma unroll
-      for (int g8 = 0; g8 < 8; ++g8) mw = max(mw, __popc((unsigned)(wm >> (8 * g8)) & 0xFFu));
+      for (int k = 1; k <= body_cap<L>(); ++k) mw = __ballot(na >= k) ? k : mw;
     }
     const int jmax = 3 * mw;
     // 2. contacts
@@ -344,7 +401,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
           }
         }
 #pragma unroll
-        for (int c2 = 0; c2 < kBodyCand; ++c2) {
+        for (int c2 = 0; c2 < body_cap<L>(); ++c2) {
           if (c2 >= mw) continue;  // columns past jmax are never read
           double Yc[6][3];
 #pragma unroll
@@ -546,7 +603,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
               for (int k = 0; k < 3; ++k) s += Wi[t][3 * i + k] * Wi[t][3 * k + j];
               const double e = dmu(i) * s * dmu(j);
 #pragma unroll
-              for (int cb = 0; cb < kBodyCand; ++cb)
+              for (int cb = 0; cb < body_cap<L>(); ++cb)
                 if (cb == sub * T + t) Lc[3 * t + i][3 * cb + j] += e;
             }
         }
@@ -652,7 +709,7 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
       const v3<double> w = mul(Rw, v3<double>{vn[0], vn[1], vn[2]});
       const v3<double> v0 = mul(Rw, v3<double>{vn[3], vn[4], vn[5]}) + cross(tw, w);
 #pragma unroll
-      for (int t = 0; t < T; ++t) {
+      for (int t = 0; t < CT; ++t) {
         const Cand& C = cd[t];
         if (C.kind < 0 || (C.kind == 1 && nct != 0.0)) continue;
         const v3<double> p = mul(Rw, v3<double>{C.pb[0], C.pb[1], C.pb[2]}) + tw;
@@ -716,20 +773,35 @@ __device__ void vs_body(const BucketArgs& a, int tid, double dt, int ccd, int n_
   }
 }
 
-template <int L> constexpr int body_lds_pitch() { return ((3 * kBodyCand / L) * kBodyRows) | 1; }
-
-template <int L>
-__global__ void __launch_bounds__(256) vs_body_kernel(BucketArgs a, double dt, int ccd, int n_steps) {
-  vs_body<L>(a, blockIdx.x * blockDim.x + threadIdx.x, dt, ccd, n_steps, (double*)GP_DYN_LDS);
+// doubles of a lane's LDS row, and LDS bytes of a workgroup
+template <int L> constexpr int body_lds_pitch() { return ((3 * body_cap<L>() / L) * 3 * body_cap<L>()) | 1; }
+template <int L> constexpr unsigned body_lds(int block) {
+  return (unsigned)((body_lds_pitch<L>() * block + block / L * kStash) * sizeof(double));
 }
 
 template <int L>
-int launch_l(const BucketArgs& a, double dt, int ccd, int n_steps, int block, hipStream_t s) {
-  const long threads = (long)a.B * L;
-  dim3 blk(block), grid((unsigned)((threads + block - 1) / block));
-  const unsigned lds = (unsigned)((body_lds_pitch<L>() * block + block / L * kStash) * sizeof(double));
-  hipLaunchKernelGGL((vs_body_kernel<L>), grid, blk, lds, s, a, dt, ccd, n_steps);
-  return (int)hipGetLastError();
+constexpr unsigned body_lds_bytes(int block) {
+  return L == 1 ? body_lds<1>(block) : std::max(body_lds<4>(block), body_lds<8>(block));
+}
+
+// One lane per instance
+__global__ void __launch_bounds__(256) vs_body_lane_kernel(BucketArgs a, double dt, int ccd, int n_steps) {
+  vs_body<1, false>(a, blockIdx.x * blockDim.x + threadIdx.x, 0, dt, ccd, n_steps, (double*)GP_DYN_LDS);
+}
+
+// A wave's per_wave (1 to 16) instances on 4 lanes each; then those that came to
+// more than four contacts, eight at a time, on 8 lanes each.
+__global__ void __launch_bounds__(256) vs_body_kernel(BucketArgs a, double dt, int ccd, int n_steps, int per_wave) {
+  const int tid = blockIdx.x * blockDim.x + threadIdx.x, lane = tid & 63, first = (tid >> 6) * per_wave;
+  double* const lds = (double*)GP_DYN_LDS;
+  if (lane / 4 < per_wave) vs_body<4, false>(a, first + lane / 4, lane & 3, dt, ccd, n_steps, lds);
+  // an instance's state and its rounds[] were written by this wave
+#ifdef __HIP_DEVICE_COMPILE__
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+#endif
+#pragma unroll 1
+  for (int at = 0; at < per_wave; at += 8)
+    if (at + lane / 8 < per_wave) vs_body<8, true>(a, first + at + lane / 8, lane & 7, dt, ccd, n_steps, lds);
 }
 
 }  // namespace
@@ -743,10 +815,21 @@ int launch_vs_body(const BucketArgs& a, double dt, int ccd, int n_steps, int lan
   if (block <= 0) block = kVsBodyBlock;
   if (block > 256 || block % 64 != 0) return (int)hipErrorInvalidValue;
   hipStream_t s = (hipStream_t)stream;
-  // one lane per body: its LDS row holds all 24 rows of G (4.6 KB), so 16
-  // lanes per workgroup (74 KB)
-  if (lanes == 1) return launch_l<1>(a, dt, ccd, n_steps, 16, s);
-  return launch_l<8>(a, dt, ccd, n_steps, block, s);
+  if (lanes == 1) {
+    // its LDS row holds all 24 rows of G (4.6 KB), so 16 lanes per workgroup (74 KB)
+    hipLaunchKernelGGL(vs_body_lane_kernel, dim3((a.B + 15) / 16), dim3(16), body_lds_bytes<1>(16), s, a, dt, ccd,
+                       n_steps);
+    return (int)hipGetLastError();
+  }
+  // A wave takes as long as the slowest of its instances, so while the chip
+  // has a SIMD for each they get a wave each, then as few to a wave as cover
+  // its 1,024 SIMDs once.
+  constexpr int kSimds = 1024;
+  const int per_wave = std::min(16, (a.B + kSimds - 1) / kSimds);
+  const long threads = ((long)a.B + per_wave - 1) / per_wave * 64;
+  dim3 blk(block), grid((unsigned)((threads + block - 1) / block));
+  hipLaunchKernelGGL(vs_body_kernel, grid, blk, body_lds_bytes<4>(block), s, a, dt, ccd, n_steps, per_wave);
+  return (int)hipGetLastError();
 }
 
 }  // namespace gp

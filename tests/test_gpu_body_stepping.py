@@ -1,0 +1,49 @@
+"""Velocity stepping of lone bodies, four lanes an instance and eight where more
+than four contacts touch, on the GPU: an instance gives the same bits whatever
+batch it is in (1 to 16 instances a wave, neighbours with more contacts than it
+has), and one step is the oracle's."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-5  # of the state, as test_gpu_velocity_stepping.py: the impulse program's stopping rule
+
+
+def _cubes(n, seed):
+    """Cubes of side 1 from sunk in the plane (up to 8 corners inside) to above it."""
+    rng = np.random.default_rng(seed)
+    q, v = np.zeros((n, 7)), rng.normal(0.0, 0.5, (n, 6))
+    x = rng.normal(size=(n, 4))
+    q[:, :4] = x / np.linalg.norm(x, axis=1, keepdims=True)
+    q[:, 6] = rng.uniform(-0.6, 1.0, n)
+    return q, v
+
+
+@pytest.mark.parametrize("integrator", [3, 4])
+@pytest.mark.parametrize("n", [1, 5, 1024, 1025, 3001, 15000])
+def test_single_bodies_do_not_depend_on_their_batch(gp, oracle, n, integrator):
+    from gorilla_physics_amd import batch, builders
+    st = builders.build_cube(1.0, 1.0)
+    st.add_halfspace(gp.HalfSpace.new([0.0, 0.0, 1.0], 0.0))
+    d = st.model_desc()
+    q, v = _cubes(n, n)
+    print(f"case {n} cubes, integrator {integrator}", flush=True)
+
+    def stepped(idx, steps):
+        b = batch.Batch([batch.Model(d)], [len(idx)])
+        b.set_state(q[idx].ravel(), v[idx].ravel())
+        b.step(1e-2, integrator, steps)
+        qn, vn = b.get_state()
+        return (qn.reshape(-1, 7), vn.reshape(-1, 6), b.get_vdot().reshape(-1, 6), b.collision_rounds(), b.faults())
+    every = np.arange(n)
+    some = sorted({int(i) for i in np.linspace(0, n - 1, 12)})
+    one, four = stepped(every, 1), stepped(every, 4)
+    assert (four[3] >= 1).all()
+    for i in some:
+        for got, x in zip(four, stepped(np.array([i]), 4)):
+            assert np.array_equal(got[i], x[0]), i
+        rq, rv, ro = oracle.vs_step(d, q[i], v[i], np.zeros(6), 1e-2, integrator == 4)
+        assert one[3][i] == ro, i
+        assert np.abs(one[0][i] - rq).max() <= TOL * max(1.0, np.abs(rq).max()), i
+        assert np.abs(one[1][i] - rv).max() <= TOL * max(1.0, np.abs(rv).max()), i

@@ -21,6 +21,7 @@ def _model(gp, kind):
 @pytest.mark.parametrize("kind", ["quadruped", "cube"])
 @pytest.mark.parametrize("n", [1, 65, 1024, 1025])  # the last one is past the wave kernel's range
 def test_wave_stepping_gives_the_lane_kernels_bits(gp, kind, n, integrator):
+    from gorilla_physics_amd import batch
     rng = np.random.default_rng(n)
     d = _model(gp, kind)
     q = rng.normal(0.0, 0.1, (n, d.nq))
@@ -29,7 +30,7 @@ def test_wave_stepping_gives_the_lane_kernels_bits(gp, kind, n, integrator):
     v, tau = rng.normal(0.0, 0.5, (n, d.nv)), rng.normal(0.0, 0.1, (n, d.nv))
     got = []
     for kernel in (0, 1):
-        b = gp.batch.Batch([gp.batch.Model(d)], [n], kernel=kernel)
+        b = batch.Batch([batch.Model(d)], [n], kernel=kernel)
         b.set_state(q.ravel(), v.ravel())
         b.set_tau(tau.ravel())
         b.step(1e-2, integrator, 3)
