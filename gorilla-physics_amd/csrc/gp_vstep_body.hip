@@ -68,6 +68,33 @@ template <int L> constexpr int body_cap() { return L == 4 ? 4 : kBodyCand; }
 // current q and v, v_free, the world rotation and translation
 constexpr int kStash = 7 + 6 + 7 + 6 + 6 + 9 + 3;
 
+// LDS of a workgroup: a slice for each wave (at one lane an instance, for the
+// workgroup's kLoneLanes lanes), in it each lane's row of G and then each
+// instance's parked state. The two programs of a wave use its slice in turn
+// and lay it out differently, so a slice holds the larger layout and no wave
+// touches another's: nothing orders the waves of a workgroup.
+constexpr int kLoneLanes = 16;
+template <int L> constexpr int body_slice_lanes() { return L == 1 ? kLoneLanes : 64; }
+template <int L> constexpr int body_lds_pitch() { return ((3 * body_cap<L>() / L) * 3 * body_cap<L>()) | 1; }
+template <int L> constexpr int body_layout_doubles() {
+  return body_lds_pitch<L>() * body_slice_lanes<L>() + body_slice_lanes<L>() / L * kStash;
+}
+template <int L> constexpr int body_slice_doubles() {
+  return L == 1 ? body_layout_doubles<1>() : std::max(body_layout_doubles<4>(), body_layout_doubles<8>());
+}
+// where a thread's row of G and its instance's parked state begin (doubles)
+template <int L> constexpr unsigned body_row_at(unsigned thread) {
+  constexpr unsigned lanes = body_slice_lanes<L>();
+  return thread / lanes * body_slice_doubles<L>() + thread % lanes * body_lds_pitch<L>();
+}
+template <int L> constexpr unsigned body_stash_at(unsigned thread) {
+  constexpr unsigned lanes = body_slice_lanes<L>();
+  return thread / lanes * body_slice_doubles<L>() + lanes * body_lds_pitch<L>() + thread % lanes / L * kStash;
+}
+template <int L> constexpr unsigned body_lds_bytes(int block) {
+  return (unsigned)(block / body_slice_lanes<L>() * body_slice_doubles<L>() * sizeof(double));
+}
+
 // x of the lane `O` apart (O = 1, 2, 4) in the instance's 8-lane group
 template <int O, class T> __device__ __forceinline__ T xor8(T x) { return lane_xor<O>(x); }
 template <int CTRL, int BANKS> __device__ __forceinline__ double dpp64(double old, double x) {
@@ -181,7 +208,6 @@ template <int L, bool RESUME>
 __device__ void vs_body(const BucketArgs& a, int inst, int sub, double dt, int ccd, int n_steps, double* lds) {
   constexpr int CT = kBodyCand / L;                     // candidates of a lane, c = t L + sub
   constexpr int T = body_cap<L>() / L, R = 3 * T, m = 3 * body_cap<L>();  // the program's contacts and rows
-  constexpr int pitch = (R * m) | 1;
   if (inst >= a.B) return;
   int step = 0;
   if constexpr (RESUME) {
@@ -189,7 +215,7 @@ __device__ void vs_body(const BucketArgs& a, int inst, int sub, double dt, int c
     if (left_at >= 0) return;
     step = -left_at - 1;
   }
-  double* Gs = lds + (size_t)threadIdx.x * pitch;  // this lane's rows of G: Gs[i * m + k]
+  double* Gs = lds + body_row_at<L>(threadIdx.x);  // this lane's rows of G: Gs[i * m + k]
   const int Bp = a.Bp, nb = a.nb, nc = a.nc, nh = a.nh;
   auto bpar = [&](int f) { return a.bp[(size_t)f * nb * Bp + inst]; };
   // ---- the contact candidates (the body's parameters are re-read, from
@@ -422,7 +448,7 @@ __device__ void vs_body(const BucketArgs& a, int inst, int sub, double dt, int c
       // The instance's state that outlives the interior point waits in LDS
       // meanwhile, its registers free for the program: every lane of the
       // instance holds the same bits, its first lane writes, all read back.
-      double* const stash = lds + (size_t)blockDim.x * pitch + (size_t)(threadIdx.x / L) * kStash;
+      double* const stash = lds + body_stash_at<L>(threadIdx.x);
       auto park = [&](bool back) {
         auto mv = [&](double& x, int k) {
           if (back) x = stash[k];
@@ -773,17 +799,6 @@ __device__ void vs_body(const BucketArgs& a, int inst, int sub, double dt, int c
   }
 }
 
-// doubles of a lane's LDS row, and LDS bytes of a workgroup
-template <int L> constexpr int body_lds_pitch() { return ((3 * body_cap<L>() / L) * 3 * body_cap<L>()) | 1; }
-template <int L> constexpr unsigned body_lds(int block) {
-  return (unsigned)((body_lds_pitch<L>() * block + block / L * kStash) * sizeof(double));
-}
-
-template <int L>
-constexpr unsigned body_lds_bytes(int block) {
-  return L == 1 ? body_lds<1>(block) : std::max(body_lds<4>(block), body_lds<8>(block));
-}
-
 // One lane per instance
 __global__ void __launch_bounds__(256) vs_body_lane_kernel(BucketArgs a, double dt, int ccd, int n_steps) {
   vs_body<1, false>(a, blockIdx.x * blockDim.x + threadIdx.x, 0, dt, ccd, n_steps, (double*)GP_DYN_LDS);
@@ -817,8 +832,8 @@ int launch_vs_body(const BucketArgs& a, double dt, int ccd, int n_steps, int lan
   hipStream_t s = (hipStream_t)stream;
   if (lanes == 1) {
     // its LDS row holds all 24 rows of G (4.6 KB), so 16 lanes per workgroup (74 KB)
-    hipLaunchKernelGGL(vs_body_lane_kernel, dim3((a.B + 15) / 16), dim3(16), body_lds_bytes<1>(16), s, a, dt, ccd,
-                       n_steps);
+    hipLaunchKernelGGL(vs_body_lane_kernel, dim3((a.B + kLoneLanes - 1) / kLoneLanes), dim3(kLoneLanes),
+                       body_lds_bytes<1>(kLoneLanes), s, a, dt, ccd, n_steps);
     return (int)hipGetLastError();
   }
   // A wave takes as long as the slowest of its instances, so while the chip

@@ -47,3 +47,52 @@ def test_single_bodies_do_not_depend_on_their_batch(gp, oracle, n, integrator):
         assert one[3][i] == ro, i
         assert np.abs(one[0][i] - rq).max() <= TOL * max(1.0, np.abs(rq).max()), i
         assert np.abs(one[1][i] - rv).max() <= TOL * max(1.0, np.abs(rv).max()), i
+
+
+def _groove(gp):
+    """A body with four contact points between two half-spaces that meet at a
+    right angle: 0 to 8 contacts."""
+    from gorilla_physics_amd import abi
+    from gorilla_physics_amd.mechanism import (Isometry3, ModelDesc, SpatialInertia, body_desc, contact_desc,
+                                               halfspace_desc)
+    body = body_desc(-1, abi.GP_JOINT_FLOATING, [0.0, 0.0, 1.0], Isometry3.identity(),
+                     SpatialInertia.cuboid_at(np.zeros(3), 1.0, 1.0, 1.0, 1.0, "box"))
+    points = [contact_desc(0, [x, y, -0.5], 50e3) for x in (-0.5, 0.5) for y in (-0.5, 0.5)]
+    planes = [halfspace_desc(gp.HalfSpace.new([s, 0.0, np.sqrt(0.5)], 0.0)) for s in (np.sqrt(0.5), -np.sqrt(0.5))]
+    return ModelDesc([body], points, planes)
+
+
+@pytest.mark.parametrize("integrator", [3, 4])
+@pytest.mark.parametrize("kind", ["cube", "groove"])
+@pytest.mark.parametrize("n", [7, 200, 3001])
+def test_single_bodies_do_not_depend_on_their_workgroup(gp, n, kind, integrator):
+    """Workgroups of one to four waves: an instance that touches with more than
+    four points is finished by eight lanes while its workgroup's other waves
+    may still be at the four-lane program; states, accelerations, rounds and
+    faults keep every bit of a batch of one."""
+    from gorilla_physics_amd import batch, builders
+    if kind == "cube":
+        st = builders.build_cube(1.0, 1.0)
+        st.add_halfspace(gp.HalfSpace.new([0.0, 0.0, 1.0], 0.0))
+        d = st.model_desc()
+    else:
+        d = _groove(gp)
+    q, v = _cubes(n, n + 1)
+    if kind == "groove":  # upright, from all points in both planes to above them
+        q[:, :4] = [0.0, 0.0, 0.0, 1.0]
+        q[:, 6] = np.random.default_rng(n).uniform(-0.2, 1.2, n)
+    print(f"case {n} {kind}s, workgroups of 64 to 256, integrator {integrator}", flush=True)
+
+    def stepped(idx, **kw):
+        b = batch.Batch([batch.Model(d)], [len(idx)], **kw)
+        b.set_state(q[idx].ravel(), v[idx].ravel())
+        b.step(1e-2, integrator, 4)
+        qn, vn = b.get_state()
+        return (qn.reshape(-1, 7), vn.reshape(-1, 6), b.get_vdot().reshape(-1, 6), b.collision_rounds(), b.faults())
+    every = np.arange(n)
+    got = [stepped(every, block_size=bs) for bs in (64, 128, 256)]
+    for g in got[1:]:
+        assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(got[0], g))
+    for i in sorted({int(i) for i in np.linspace(0, n - 1, 10)}):
+        for x, y in zip(got[0], stepped(np.array([i]))):
+            assert np.array_equal(x[i], y[0], equal_nan=True), i
