@@ -1700,10 +1700,10 @@ extern "C" int gp_batch_autotune(gp_batch* bt, double dt, int32_t integrator, in
   if (trial_steps < 0) return fail(GP_ERR_INVALID, "trial_steps < 0");
   const int steps = trial_steps > 0 ? trial_steps : 200;
   HIP_TRY(hipStreamSynchronize(bt->stream));
-  bool has_free = false, has_tree = false, has_fast = false;
+  bool has_free = false, has_tree = false, has_blocks = false;
   for (const Bucket& b : bt->buckets) {
     const bool fast = bucket_is_fast(bt->opts, b, integrator);
-    has_fast = has_fast || fast;
+    has_blocks = has_blocks || fast || bucket_aux_tree(bt->opts, b, integrator);
     has_free = has_free || (fast && b.fast_topo == TOPO_FREE);
     has_tree = has_tree || (fast && b.fast_topo == TOPO_QUAD);
   }
@@ -1713,11 +1713,12 @@ extern "C" int gp_batch_autotune(gp_batch* bt, double dt, int32_t integrator, in
   if (st) return st;
   gp_batch_opts best = user;
   best.use_graph = 0;  // trials time the launches themselves
-  // spell out the defaults, so that no candidate re-measures the starting point
+  // spell out the defaults, so that no candidate re-measures the starting point.
+  // A workgroup size of 0 stays 0: each kernel has its own default, and a size
+  // that no trial beat is not put in its place for the kernels of later calls
   if (best.lanes_per_mech == 0) best.lanes_per_mech = 4;
   if (best.lanes_per_tree == 0) best.lanes_per_tree = 4;
   if (best.steps_per_launch == 0) best.steps_per_launch = 100;
-  if (best.block_size == 0) best.block_size = grouped_count(bt, integrator) > 0 ? 128 : 256;
   double best_t = 0;
   auto run = [&](const gp_batch_opts& o, double* t) {
     int e = gp_batch_set_opts(bt, &o);
@@ -1732,8 +1733,8 @@ extern "C" int gp_batch_autotune(gp_batch* bt, double dt, int32_t integrator, in
   const Dim dims[] = {
       {&gp_batch_opts::lanes_per_mech, {1, 2, 4, 8}, has_free},
       {&gp_batch_opts::lanes_per_tree, {1, 4}, has_tree && integrator == GP_SEMI_IMPLICIT_EULER},
-      {&gp_batch_opts::block_size, {64, 128, 256}, has_fast},
-      {&gp_batch_opts::steps_per_launch, {25, 50, 100, 200}, has_fast},
+      {&gp_batch_opts::block_size, {64, 128, 256}, has_blocks},
+      {&gp_batch_opts::steps_per_launch, {25, 50, 100, 200}, has_blocks},
   };
   for (const Dim& d : dims) {
     if (st || !d.used) continue;

@@ -1,0 +1,118 @@
+// Checks of the library's host side against the stand-in for the HIP runtime,
+// where what a call asks of the device can be written down: no kernel of a
+// compiled topology or tree runs, its launch is recorded instead.
+//
+//   runtime_host <check>
+//
+// Prints what it saw and returns 1 if that is wrong.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "../../include/gorilla_amd.h"
+#include "../../gorilla-physics_amd/csrc/gp_internal.h"
+
+namespace {
+struct FastLaunch { int topo, n_steps, block; };
+std::vector<FastLaunch> fast_launches;
+}  // namespace
+
+namespace gp {
+int fast_topology_id(int, const int*, const int*, int) { return -1; }
+int launch_fast_step(int topo, int, const BucketArgs&, double, int n_steps, int block, void*) {
+  fast_launches.push_back({topo, n_steps, block});
+  return hipSuccess;
+}
+int launch_fast_rk_step(int, int, int, const BucketArgs&, double, int, int, void*) { return hipErrorNotSupported; }
+int launch_grouped_step(const GroupTable*, int, int, double, int, int, void*) { return hipErrorNotSupported; }
+}  // namespace gp
+
+static void need(bool c, const char* what) {
+  if (!c) {
+    std::printf("%s (%s)\n", what, gp_last_error());
+    std::exit(1);
+  }
+}
+
+// A floating body with a revolute one on it, a contact point and a plane: a
+// tree that no compiled topology covers.
+static gp_model* small_tree() {
+  gp_body_desc body[2] = {};
+  for (int i = 0; i < 2; ++i) {
+    body[i].parent = i - 1;
+    body[i].jtype = i == 0 ? GP_JOINT_FLOATING : GP_JOINT_REVOLUTE;
+    body[i].axis[2] = 1.0;
+    body[i].x_tree_quat[3] = 1.0;
+    for (int k = 0; k < 3; ++k) body[i].moment[k] = 1.0;
+    body[i].mass = 1.0;
+  }
+  gp_contact_desc contact{};
+  contact.k = 50e3;
+  gp_halfspace_desc plane{};
+  plane.normal[2] = 1.0;
+  plane.alpha = 0.9;
+  plane.mu = 0.5;
+  gp_model_desc d{};
+  d.n_bodies = 2;
+  d.bodies = body;
+  d.n_contacts = 1;
+  d.contacts = &contact;
+  d.n_halfspaces = 1;
+  d.halfspaces = &plane;
+  d.gravity = 9.81;
+  gp_model* m = nullptr;
+  need(gp_model_create(&d, &m) == GP_OK, "gp_model_create");
+  return m;
+}
+
+static gp_batch* batch_of(gp_model* m, int64_t n, gp_batch_opts o) {
+  o.separate_launches = 1;
+  gp_batch* b = nullptr;
+  need(gp_batch_create(&m, &n, 1, &o, &b) == GP_OK, "gp_batch_create");
+  return b;
+}
+
+// The autotuner starts from the options that gp_step uses without it, tries
+// sizes where a kernel has one, and adopts none that it has not measured to be
+// faster (the stand-in's events measure nothing).
+static void autotune() {
+  gp_model* m = small_tree();
+  for (int kernel : {GP_KERNEL_AUTO, GP_KERNEL_PLAIN}) {
+    gp_batch_opts o{};
+    o.kernel = kernel;
+    gp_batch* b = batch_of(m, 3, o);
+    fast_launches.clear();
+    gp_batch_opts chosen{};
+    double ms = -1.0;
+    need(gp_batch_autotune(b, 1e-3, GP_SEMI_IMPLICIT_EULER, 50, &chosen, &ms) == GP_OK, "gp_batch_autotune");
+    need(chosen.block_size == 0, "a workgroup size was adopted without a faster trial");
+    const bool tree = kernel == GP_KERNEL_AUTO;
+    need(tree == !fast_launches.empty(), "the tree kernel runs exactly by the automatic choice");
+    if (tree) {
+      need(fast_launches[0].block == 0, "the first trial is not the default's");
+      for (int size : {64, 128, 256}) {
+        bool tried = false;
+        for (const FastLaunch& l : fast_launches) tried = tried || l.block == size;
+        need(tried, "a workgroup size was not tried");
+      }
+      bool split = false;
+      for (const FastLaunch& l : fast_launches) split = split || l.n_steps == 25;
+      need(split, "fewer steps a launch were not tried");
+    }
+    gp_batch_destroy(b);
+  }
+  gp_model_destroy(m);
+}
+
+int main(int argc, char** argv) {
+  need(argc == 2, "usage: runtime_host <check>");
+  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}};
+  for (const auto& c : checks)
+    if (!std::strcmp(argv[1], c.name)) {
+      c.f();
+      std::printf("%s ok\n", c.name);
+      return 0;
+    }
+  need(false, "no such check");
+}
