@@ -150,6 +150,25 @@ void chain_frames(gp_model& m, int first, std::vector<M>& Al) {
   }
 }
 
+// Makes a device the calling thread's current one for a scope. The null stream
+// is the current device's, so a call that uses it makes the batch's device
+// current: the thread may have another one.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) {
+    int now = 0;
+    if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) before_ = now;
+  }
+  ~OnDevice() {
+    if (before_ >= 0) (void)hipSetDevice(before_);
+  }
+  OnDevice(const OnDevice&) = delete;
+  OnDevice& operator=(const OnDevice&) = delete;
+
+ private:
+  int before_ = -1;
+};
+
 uint64_t fnv(uint64_t h, int64_t x) {
   for (int k = 0; k < 8; ++k) {
     h ^= (uint64_t)((x >> (8 * k)) & 0xff);
@@ -846,6 +865,7 @@ int gp_batch_create(gp_model* const* models, const int64_t* counts, int32_t n_mo
     if (st) return st;
     int ndev = 0;
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev < 1) return fail(GP_ERR_DEVICE, "no HIP device");
+    HIP_TRY(hipGetDevice(&bt->device));
     // group instances by topology signature (first-seen order)
     std::map<uint64_t, int> sig_bucket;
     std::vector<std::vector<const gp_model*>> lanes;
@@ -1011,6 +1031,7 @@ static int transfer_by_bucket(gp_batch* bt, const double* hq, const double* hv, 
 // 1,462 / 277; get_state of 1 31 / 18, of 65,536 946 / 502.
 static int transfer(gp_batch* bt, const double* hq, const double* hv, double* oq, double* ov, bool to_dev,
                     int which /*0 state, 1 tau, 2 vdot, 3 tau_tmp*/) {
+  const OnDevice on(bt->device);
   double* flat = bt->d_flat;
   const size_t values = (size_t)(which == 0 ? bt->qoff.back() + bt->voff.back() : bt->voff.back());
   const bool few = to_dev && bt->buckets.size() == 1 && values <= (which == 0 ? 256u : 32768u);
@@ -1424,6 +1445,7 @@ static int query_plan(gp_batch* bt, bool* tree, std::vector<int>* rest) {
 
 int gp_dynamics(gp_batch* bt, const double* tau, double* vdot) {
   if (!bt || !vdot) return fail(GP_ERR_INVALID, "null argument");
+  const OnDevice on(bt->device);
   int st;
   if (tau && (st = transfer(bt, nullptr, tau, nullptr, nullptr, true, 3))) return st;
   bool tree = false;
@@ -1447,6 +1469,7 @@ int gp_dynamics(gp_batch* bt, const double* tau, double* vdot) {
 // M (instance-major, each nv_i x nv_i row-major) or c - tau_c (the v
 // flattening) of every instance at the batch's state
 static int joint_space_terms(gp_batch* bt, double* Mh, double* ch) {
+  const OnDevice on(bt->device);
   bool tree = false;
   std::vector<int> rest;
   int st = query_plan(bt, &tree, &rest);

@@ -119,6 +119,7 @@ struct gp_batch {
   std::vector<int64_t> qoff, voff;
   std::vector<int> inst_bucket, inst_lane;
   gp_batch_opts opts{};
+  int device = 0;  // whose memory the batch is in (the creating thread's current one)
   hipStream_t stream = nullptr;
   // a caller's own stream has carried this batch's work since the last
   // gp_batch_sync (which then waits for the whole device)

@@ -74,12 +74,17 @@ inline hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { s
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
 inline hipError_t hipMemset(void* d, int v, size_t n) { std::memset(d, v, n); return hipSuccess; }
 inline hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
-inline hipError_t hipStreamCreate(hipStream_t* s) { *s = nullptr; return hipSuccess; }
+inline char gp_host_stream_token;  // what every created stream points at: not the null stream
+inline hipError_t hipStreamCreate(hipStream_t* s) { *s = (hipStream_t)&gp_host_stream_token; return hipSuccess; }
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
 inline hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
-inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+// The calling thread's current device, and the one that the last launch on
+// the null stream went to (a number only: there is one memory)
+inline thread_local int gp_host_device = 0, gp_host_null_stream_device = -1;
+inline hipError_t hipGetDevice(int* d) { *d = gp_host_device; return hipSuccess; }
+inline hipError_t hipSetDevice(int d) { gp_host_device = d; return hipSuccess; }
 template <class T> inline hipError_t hipGetSymbolAddress(void** p, T* symbol) { *p = (void*)symbol; return hipSuccess; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
 inline const char* hipGetErrorString(hipError_t) { return "host build"; }
@@ -179,6 +184,7 @@ inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v 
     void* gp_lds_ = nullptr;                                                 \
     if (gp_sh_) (void)hipMalloc(&gp_lds_, gp_sh_);                           \
     gp_host_dyn_lds = (unsigned char*)gp_lds_;                               \
+    if (!(hipStream_t)(stream)) gp_host_null_stream_device = gp_host_device; \
     for (unsigned gp_bx = 0; gp_bx < gp_g_.x; ++gp_bx)                       \
       for (unsigned gp_tx = 0; gp_tx < gp_b_.x; ++gp_tx) {                   \
         blockIdx.x = gp_bx;                                                  \

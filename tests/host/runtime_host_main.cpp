@@ -66,6 +66,24 @@ static gp_model* small_tree() {
   return m;
 }
 
+// A lone body on a joint of this type.
+static gp_model* lone_body(int jtype) {
+  gp_body_desc body{};
+  body.parent = -1;
+  body.jtype = jtype;
+  body.axis[2] = 1.0;
+  body.x_tree_quat[3] = 1.0;
+  for (int k = 0; k < 3; ++k) body.moment[k] = 1.0;
+  body.mass = 1.0;
+  gp_model_desc d{};
+  d.n_bodies = 1;
+  d.bodies = &body;
+  d.gravity = 9.81;
+  gp_model* m = nullptr;
+  need(gp_model_create(&d, &m) == GP_OK, "gp_model_create");
+  return m;
+}
+
 static gp_batch* batch_of(gp_model* m, int64_t n, gp_batch_opts o) {
   o.separate_launches = 1;
   gp_batch* b = nullptr;
@@ -105,9 +123,42 @@ static void autotune() {
   gp_model_destroy(m);
 }
 
+// Host calls reach the batch's device whatever device the calling thread has
+// made current, and leave that as it was.
+static void device() {
+  gp_model* m[2] = {lone_body(GP_JOINT_FLOATING), lone_body(GP_JOINT_REVOLUTE)};
+  const int64_t n[2] = {3, 2};
+  gp_batch* b = nullptr;
+  need(hipSetDevice(2) == hipSuccess && gp_batch_create(m, n, 2, nullptr, &b) == GP_OK, "gp_batch_create");
+  need(hipSetDevice(5) == hipSuccess, "hipSetDevice");
+  const int nq = 3 * 7 + 2, nv = 3 * 6 + 2, nm = 3 * 36 + 2;
+  std::vector<double> q(nq, 0.5), v(nv, 0.25), out(nm), out2(nm);
+  auto check = [&](int st, const char* call) {
+    need(st == GP_OK, call);
+    int now = -1;
+    need(hipGetDevice(&now) == hipSuccess && now == 5, "the caller's device was changed");
+    if (gp_host_null_stream_device != 2) {
+      std::printf("%s launched on device %d, the batch is on 2\n", call, gp_host_null_stream_device);
+      std::exit(1);
+    }
+    gp_host_null_stream_device = -1;
+  };
+  check(gp_batch_set_state(b, q.data(), v.data()), "gp_batch_set_state");
+  check(gp_batch_set_tau(b, v.data()), "gp_batch_set_tau");
+  check(gp_batch_get_state(b, out.data(), out2.data()), "gp_batch_get_state");
+  check(gp_dynamics(b, nullptr, out.data()), "gp_dynamics");
+  check(gp_dynamics(b, v.data(), out.data()), "gp_dynamics");
+  check(gp_batch_get_vdot(b, out.data()), "gp_batch_get_vdot");
+  check(gp_mass_matrix(b, out.data()), "gp_mass_matrix");
+  check(gp_dynamics_bias(b, out.data()), "gp_dynamics_bias");
+  gp_batch_destroy(b);
+  for (gp_model* x : m) gp_model_destroy(x);
+  need(hipSetDevice(0) == hipSuccess, "hipSetDevice");
+}
+
 int main(int argc, char** argv) {
   need(argc == 2, "usage: runtime_host <check>");
-  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}};
+  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}, {"device", device}};
   for (const auto& c : checks)
     if (!std::strcmp(argv[1], c.name)) {
       c.f();
