@@ -1365,8 +1365,29 @@ int gp_batch_get_vdot(gp_batch* bt, double* vdot) {
   return transfer(bt, nullptr, nullptr, nullptr, vdot, false, 2);
 }
 
+// Whether gp_dynamics of a bucket that the tree kernel takes is faster there
+// (one body per lane) than in the plain kernel (one instance per lane): the
+// estimate of both in us. A wave of the tree kernel goes through its levels
+// one after the other and loads a line per body and field, which instances of
+// many bodies share less, 2,048 waves at a time; the plain kernel's time is its
+// bodies' chain of dependent scratch accesses, then their bytes. So long chains in large batches are the plain
+// kernel's. Tree / plain kernel, us, at 4,096, 16,384 and 65,536 instances:
+// chains of 12 bodies 31 / 136, 82 / 150, 208 / 285; of 16 41 / 185, 114 / 205,
+// 367 / 402; of 22 80 / 252, 230 / 291, 838 / 521; of 32 167 / 376, 364 / 501,
+// 1,299 / 762; of 40 221 / 470, 760 / 645, 2,852 / 940; of 64 432 / 702, 1,306 /
+// 1,033, 4,965 / 1,500; trees of 64 bodies in 4 levels 105 / 730, 307 / 990, 1,410
+// / 1,420. Of 160 sizes tried the estimate takes the slower one at one, by 4 %
+// (32,768 chains of 24).
+static bool tree_dynamics_faster(const Bucket& b) {
+  const double waves = (double)fast_threads(TOPO_TREE, b.B, b.nb) / 64.0, bodies = 64 / b.nb * b.nb;
+  const double tree = waves / 2048.0 * (bodies * (0.1 + b.nb / 130.0) + 2.0 * (b.max_depth + 1));
+  const double plain = b.nb * (11.0 + 2.8e-4 * b.B);
+  return tree <= plain;
+}
+
 // The queries' table over the buckets that the tree kernel takes (no spring
-// contacts, at most 8 children a body) and the list of the others.
+// contacts, at most 8 children a body), first those whose accelerations it
+// computes too, and the lists of the others.
 static int ensure_query(gp_batch* bt) {
   if (bt->query_built) return GP_OK;
   bt->moff.assign(bt->n_inst + 1, 0);
@@ -1374,28 +1395,35 @@ static int ensure_query(gp_batch* bt) {
     const int64_t nv = bt->voff[i + 1] - bt->voff[i];
     bt->moff[i + 1] = bt->moff[i] + nv * nv;
   }
-  std::vector<QueryEntry> table;
-  std::vector<int64_t> moff;  // by entry and lane
-  std::vector<int> other;
-  unsigned blocks = 0;
-  int lds = 0;
+  std::vector<int> order, long_chains, other;  // buckets
+  std::vector<size_t> off_at;                  // each bucket's first entry of the lanes' offsets
   size_t at = 0;
   for (size_t k = 0; k < bt->buckets.size(); ++k) {
     const Bucket& b = bt->buckets[k];
-    if (b.nsp == 0 && aux_tree_ok(b.nb, b.parent.data())) {
-      QueryEntry e{};
-      e.a = bucket_args(b, b.nb, nullptr);
-      e.tau_tmp = b.d_tau_tmp;
-      e.voff = (const int64_t*)bt->d_block + at + b.B;
-      e.first = blocks;
-      blocks += (unsigned)(fast_threads(TOPO_TREE, b.B, b.nb) / 64);
-      lds = std::max(lds, query_lds_per_wave(b.nb, b.nq - b.nv));
-      for (int l = 0; l < b.B; ++l) moff.push_back(bt->moff[b.inst[l]]);
-      table.push_back(e);
-    } else {
-      other.push_back((int)k);
-    }
+    if (b.nsp > 0 || !aux_tree_ok(b.nb, b.parent.data())) other.push_back((int)k);
+    else if (tree_dynamics_faster(b)) order.push_back((int)k);
+    else long_chains.push_back((int)k);
+    off_at.push_back(at);
     at += 2 * (size_t)b.B;
+  }
+  const size_t both = order.size();
+  order.insert(order.end(), long_chains.begin(), long_chains.end());
+  std::vector<QueryEntry> table;
+  std::vector<int64_t> moff;  // by entry and lane
+  unsigned blocks = 0, both_blocks = 0;
+  int lds = 0;
+  for (size_t i = 0; i < order.size(); ++i) {
+    const Bucket& b = bt->buckets[order[i]];
+    QueryEntry e{};
+    e.a = bucket_args(b, b.nb, nullptr);
+    e.tau_tmp = b.d_tau_tmp;
+    e.voff = (const int64_t*)bt->d_block + off_at[order[i]] + b.B;
+    e.first = blocks;
+    blocks += (unsigned)(fast_threads(TOPO_TREE, b.B, b.nb) / 64);
+    if (i < both) both_blocks = blocks;
+    lds = std::max(lds, query_lds_per_wave(b.nb, b.nq - b.nv));
+    for (int l = 0; l < b.B; ++l) moff.push_back(bt->moff[b.inst[l]]);
+    table.push_back(e);
   }
   if (!table.empty()) {
     const size_t tb = table.size() * sizeof(QueryEntry);
@@ -1418,7 +1446,10 @@ static int ensure_query(gp_batch* bt) {
   }
   bt->query_n = (int)table.size();
   bt->query_blocks = blocks;
+  bt->query_dyn_n = (int)both;
+  bt->query_dyn_blocks = both_blocks;
   bt->query_lds = lds;
+  bt->query_long = std::move(long_chains);
   bt->query_other = std::move(other);
   bt->query_built = true;
   return GP_OK;
@@ -1426,11 +1457,12 @@ static int ensure_query(gp_batch* bt) {
 
 // Buckets that a query visits one by one with the one-instance-per-lane
 // kernels: all of them with GP_KERNEL_PLAIN, else those that the tree kernel
-// does not take. One launch over all the others with one body per lane was
-// faster at every size tried (us a call, host arrays, one instance per lane
-// against one body per lane): M of one quadruped 174 / 26, of 8,192 15,919 /
-// 756; c of 8,192 1,310 / 79; vdot of one 12-joint arm 125 / 36, of 65,536
-// 650 / 597.
+// does not take (gp_dynamics: see tree_dynamics_faster as well). For M and c one
+// launch over all the others with one body per lane was faster at every size
+// tried (us a call, host arrays, one instance per lane against one body per lane):
+// M of one quadruped 174 / 26, of 8,192 15,919 / 756, of 16,384 24-body chains
+// 67,846 / 4,771; c of 8,192 quadrupeds 1,310 / 79, of 65,536 64-body chains
+// 540,614 / 5,480.
 static int query_plan(gp_batch* bt, bool* tree, std::vector<int>* rest) {
   *tree = bt->opts.kernel != GP_KERNEL_PLAIN;
   if (!*tree) {
@@ -1452,8 +1484,14 @@ int gp_dynamics(gp_batch* bt, const double* tau, double* vdot) {
   std::vector<int> rest;
   if ((st = query_plan(bt, &tree, &rest))) return st;
   if (tree) {
+    // the long chains by the plain kernel, unless there is no room for its scratch
+    bool room = true;
+    for (int k : bt->query_long) room = room && bucket_ensure_scratch(bt->buckets[k]) == GP_OK;
+    if (room) rest.insert(rest.end(), bt->query_long.begin(), bt->query_long.end());
+    else (void)hipGetLastError();
     // on the null stream, which waits for the batch's
-    int e = launch_tree_dynamics(bt->d_query, bt->query_n, bt->query_blocks, bt->query_lds, tau ? 0 : 1, nullptr);
+    int e = launch_tree_dynamics(bt->d_query, room ? bt->query_dyn_n : bt->query_n,
+                                 room ? bt->query_dyn_blocks : bt->query_blocks, bt->query_lds, tau ? 0 : 1, nullptr);
     if (e) return fail(GP_ERR_DEVICE, "dynamics launch: %s", hipGetErrorString((hipError_t)e));
   }
   for (int k : rest) {

@@ -144,12 +144,14 @@ struct gp_batch {
   double* d_flat = nullptr;  // flat staging array of the host transfers, or null
   void* d_block = nullptr;   // the allocation that holds these and the lanes' offsets
   // The queries' table (gp_dynamics, gp_mass_matrix, gp_dynamics_bias), built
-  // on first use: the buckets that the tree kernel takes, and the others' indices
+  // on first use: the buckets that the tree kernel takes, the first query_dyn_n
+  // for gp_dynamics too, and the indices of the long ones that gp_dynamics
+  // leaves to the plain kernel and of those that it does not take
   bool query_built = false;
   gp::QueryEntry* d_query = nullptr;
-  int query_n = 0, query_lds = 0;
-  unsigned query_blocks = 0;
-  std::vector<int> query_other;
+  int query_n = 0, query_dyn_n = 0, query_lds = 0;
+  unsigned query_blocks = 0, query_dyn_blocks = 0;
+  std::vector<int> query_long, query_other;
   std::vector<int64_t> moff;  // each instance's offset in the mass matrices (n + 1)
   double* d_terms = nullptr;  // their results, kept while small (kTermsKept)
   size_t terms_cap = 0;

@@ -109,3 +109,41 @@ def test_terms_builders_with_fixed_joints(gp, oracle):
     w = dict(models=descs, counts=[1] * len(descs), q=np.concatenate(qs), v=v, tau=rng.normal(0.0, 0.5, v.size),
              dt=1e-3)
     _check(gp, oracle, w, "builders")
+
+
+def test_dynamics_of_long_chains_in_large_batches(gp, oracle):
+    """vdot, M and c of a batch whose long chains' accelerations are the plain
+    kernel's (33 bodies, 16,384 instances: past the line where one body per lane
+    is the slower one) beside buckets whose are not, before and after it in the
+    batch: the plain kernel's bits for those chains, M and c of every bucket
+    within 1e-10 of the oracle, and M vdot + c = tau to one rounding for each of a
+    joint's some 640 operations (the oracle's LU of such an M, of condition 1e7
+    and more, is itself 1e-9 off)."""
+    from gorilla_physics_amd import batch, workloads
+    rng = np.random.default_rng(3)
+    descs = [workloads.arms(1, seed=k, dof=nb)["models"][0] for k, nb in enumerate((20, 33, 64))]
+    counts = [3, 16384, 2]
+    inst = _descs(dict(models=descs, counts=counts))
+    q = rng.normal(0.0, 0.3, sum(d.nv for d in inst))
+    v, tau = rng.normal(0.0, 0.3, q.size), rng.normal(0.0, 0.1, q.size)
+    at = np.concatenate([[0], np.cumsum([d.nv for d in inst])])
+    print(f"case long chains: {len(inst)} instances", flush=True)
+    got = []
+    for kernel in (0, 1):
+        b = batch.Batch([batch.Model(d) for d in descs], counts, kernel=kernel)
+        b.set_state(q, v)
+        b.set_tau(tau)
+        got.append((b.dynamics(), b.dynamics(2.0 * tau)))
+        assert not b.faults().any()
+        if kernel == 0:
+            Ms, c = b.mass_matrices(), b.dynamics_bias()
+    chains = slice(at[3], at[3 + 16384])
+    for x, y in zip(*got):
+        assert np.array_equal(x[chains], y[chains])
+    for i in (0, 2, 3, 4, 66, 4000, 16386, 16387, 16388):
+        s = slice(at[i], at[i + 1])
+        Mr, cr = oracle.mass_matrix(inst[i], q[s], v[s])
+        assert rel_err(Ms[i], Mr) <= TOL and rel_err(c[s], cr) <= TOL, i
+        for a, t in ((got[0][0][s], tau[s]), (got[0][1][s], 2.0 * tau[s])):
+            size = np.abs(Mr) @ np.abs(a) + np.abs(cr) + np.abs(t)
+            assert np.abs(Mr @ a + cr - t).max() <= 640 * a.size * 2.0 ** -53 * size.max(), i
