@@ -681,6 +681,18 @@ static int vs_body_candidate_count(const Bucket& b) {
   return P <= kVsBodyMaxCandidates ? P : -1;
 }
 
+static bool bucket_vs_wave(const gp_batch_opts& o, const Bucket& b) {
+  return o.kernel != GP_KERNEL_PLAIN && vs_wave_ok(b.B, b.nb, b.nq, b.nv, b.nc, b.nh, b.ns);
+}
+
+// Whether a bucket's steps run one of the kernels that keep their working set in
+// device scratch: the plain one and velocity stepping with one instance per lane.
+static bool bucket_uses_scratch(const gp_batch_opts& o, const Bucket& b, int integrator) {
+  if (is_velocity_stepping(integrator))
+    return !(o.kernel != GP_KERNEL_PLAIN && vs_body_candidate_count(b) >= 0) && !bucket_vs_wave(o, b);
+  return !bucket_is_fast(o, b, integrator) && !bucket_aux_tree(o, b, integrator);
+}
+
 // Every bucket's launches for n_steps steps. scratch_override: where the
 // runtime-topology and velocity-stepping kernels keep their per-lane working
 // set (nullptr: each bucket's own buffer, allocated on first use; else that
@@ -725,11 +737,11 @@ static int batch_launch_all(gp_batch* bt, double dt, int integrator, int n_steps
         }
         continue;
       }
-      int st = scratch_override ? GP_OK : bucket_ensure_scratch(b);
+      const bool wave = bucket_vs_wave(o, b);
+      int st = wave || scratch_override ? GP_OK : bucket_ensure_scratch(b);
       if (st) return st;
       BucketArgs a = bucket_args(b, 1, nullptr);
       if (scratch_override) a.scratch = scratch_override;
-      const bool wave = o.kernel != GP_KERNEL_PLAIN && vs_wave_ok(b.B, b.nb, b.nq, b.nv, b.nc, b.nh, b.ns);
       for (int done = 0; done < n_steps; done += spl) {
         const int n = std::min(spl, n_steps - done);
         int e = wave ? launch_vs_wave(a, dt, ccd, n, s) : launch_vs_step(a, dt, ccd, n, s);
@@ -1237,7 +1249,7 @@ static int chunk_graph(gp_batch* bt, double dt, int integrator, int steps, hipSt
   if (it == bt->graphs.end()) {
     // bucket scratch must exist before capture (no allocation inside a graph)
     for (Bucket& b : bt->buckets) {
-      int st = bucket_ensure_scratch(b);
+      int st = bucket_uses_scratch(bt->opts, b, integrator) ? bucket_ensure_scratch(b) : GP_OK;
       if (st) return st;
     }
     int64_t n = 0;

@@ -156,9 +156,44 @@ static void device() {
   need(hipSetDevice(0) == hipSuccess, "hipSetDevice");
 }
 
+// Steps of kernels that keep nothing in device scratch (trees, velocity stepping
+// of a lone body or with one instance per wave) allocate none, nor does the
+// preparation of their graphs; the plain kernel's do.
+static void scratch() {
+  gp_model* tree = small_tree();
+  gp_model* body = lone_body(GP_JOINT_FLOATING);
+  const struct { gp_model* m; int kernel, integrator, graph; bool uses; const char* what; } cases[] = {
+      {tree, GP_KERNEL_AUTO, GP_VELOCITY_STEPPING, 0, false, "velocity stepping, one instance per wave"},
+      {tree, GP_KERNEL_PLAIN, GP_VELOCITY_STEPPING, 0, true, "velocity stepping, one instance per lane"},
+      {tree, GP_KERNEL_AUTO, GP_SEMI_IMPLICIT_EULER, 1, false, "graph of a tree's steps"},
+      {tree, GP_KERNEL_PLAIN, GP_SEMI_IMPLICIT_EULER, 1, true, "graph of the plain kernel's steps"},
+      {tree, GP_KERNEL_AUTO, GP_RUNGE_KUTTA_4, 1, true, "graph of a tree's Runge-Kutta steps"},
+      {body, GP_KERNEL_AUTO, GP_CCD_VELOCITY_STEPPING, 1, false, "graph of a lone body's velocity stepping"},
+      {tree, GP_KERNEL_AUTO, GP_VELOCITY_STEPPING, 1, false, "graph of velocity stepping, one instance per wave"},
+  };
+  for (const auto& c : cases) {
+    gp_batch_opts o{};
+    o.kernel = c.kernel;
+    o.use_graph = c.graph;
+    gp_batch* b = batch_of(c.m, 3, o);
+    const size_t before = gp_host_malloc_calls;
+    if (c.graph) (void)gp_step_prepare(b, 1e-3, c.integrator, 2, nullptr);  // the stand-in captures no graph
+    else need(gp_step(b, 1e-3, c.integrator, 2, nullptr) == GP_OK, "gp_step");
+    // a launch of the stand-in allocates its LDS
+    const bool allocated = gp_host_malloc_calls - before > (c.graph || c.kernel == GP_KERNEL_PLAIN ? 0u : 1u);
+    if (allocated != c.uses) {
+      std::printf("%s: %s scratch\n", c.what, allocated ? "allocates" : "has no");
+      std::exit(1);
+    }
+    gp_batch_destroy(b);
+  }
+  gp_model_destroy(tree);
+  gp_model_destroy(body);
+}
+
 int main(int argc, char** argv) {
   need(argc == 2, "usage: runtime_host <check>");
-  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}, {"device", device}};
+  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}, {"device", device}, {"scratch", scratch}};
   for (const auto& c : checks)
     if (!std::strcmp(argv[1], c.name)) {
       c.f();
