@@ -157,3 +157,31 @@ def test_so101_workload_shape_and_prefix(gp):
     assert a["counts"] == [5] and a["models"][0].nq == 6 and a["q"].size == 30 and a["integrator"] == 2
     for key in ("q", "v", "tau"):
         assert np.array_equal(a[key], b[key][:30])
+
+
+def test_a_kept_mass_matrix_keeps_little_else(gp):
+    """Batch.mass_matrices over runs of instances of 7, 0, 3 and 100 values a
+    side: every matrix its own values, square and writable, and what one of them
+    keeps alive is itself or at most 64 KiB, not the whole batch's."""
+    import ctypes
+    from gorilla_physics_amd import batch
+    sizes = np.array([7] * 5000 + [0] * 3 + [3] * 2000 + [100] * 2 + [7])
+    values = np.random.default_rng(0).normal(size=int((sizes ** 2).sum()))
+
+    class Lib:
+        def gp_mass_matrix(self, handle, out):
+            ctypes.memmove(out, values.ctypes.data, values.nbytes)
+            return 0
+    b = batch.Batch.__new__(batch.Batch)
+    b.handle, b.lib = None, Lib()
+    b.offsets = lambda: (None, np.concatenate([[0], np.cumsum(sizes)]))
+    got = b.mass_matrices()
+    assert [m.shape for m in got] == [(n, n) for n in sizes]
+    assert np.array_equal(np.concatenate([m.reshape(-1) for m in got]), values)
+    for m in got:
+        kept = m
+        while kept.base is not None:
+            kept = kept.base
+        assert m.flags.writeable and kept.nbytes <= max(64 << 10, m.nbytes)
+    got[0][:] = 0.0
+    assert np.array_equal(got[1].reshape(-1), values[49:98])
