@@ -929,21 +929,12 @@ int gp_batch_create(gp_model* const* models, const int64_t* counts, int32_t n_mo
       bt->voff[i + 1] = bt->voff[i] + b.nv;
     }
     // The transfers' block, one allocation and one copy: each lane's offsets into
-    // the flattened arrays (q, then v, bucket after bucket), the tables (state,
-    // torques, accelerations, gp_dynamics' torques), and a flat staging array
-    // (one q and one v) for the host calls, which do without it if it does not fit.
+    // the flattened arrays (q, then v, bucket after bucket) and the tables (state,
+    // torques, accelerations, gp_dynamics' torques).
     const size_t off_bytes = 2 * (size_t)inst * sizeof(int64_t);
     const size_t table_bytes = 5 * bt->buckets.size() * sizeof(XferEntry);
-    const size_t head = (off_bytes + table_bytes + 255) / 256 * 256;
-    const size_t staging = (size_t)(bt->qoff.back() + bt->voff.back()) * sizeof(double);
-    const bool fits = hipMalloc(&bt->d_block, head + staging) == hipSuccess;
-    if (!fits) {
-      (void)hipGetLastError();
-      bt->d_block = nullptr;
-      HIP_TRY(hipMalloc(&bt->d_block, head));
-    }
+    HIP_TRY(hipMalloc(&bt->d_block, off_bytes + table_bytes));
     char* block = (char*)bt->d_block;
-    bt->d_flat = fits && staging ? (double*)(block + head) : nullptr;
     bt->d_xfer = (XferEntry*)(block + off_bytes);
     std::vector<char> h(off_bytes + table_bytes, 0);
     int64_t* off = (int64_t*)h.data();
@@ -1044,9 +1035,17 @@ static int transfer_by_bucket(gp_batch* bt, const double* hq, const double* hv, 
 static int transfer(gp_batch* bt, const double* hq, const double* hv, double* oq, double* ov, bool to_dev,
                     int which /*0 state, 1 tau, 2 vdot, 3 tau_tmp*/) {
   const OnDevice on(bt->device);
-  double* flat = bt->d_flat;
   const size_t values = (size_t)(which == 0 ? bt->qoff.back() + bt->voff.back() : bt->voff.back());
   const bool few = to_dev && bt->buckets.size() == 1 && values <= (which == 0 ? 256u : 32768u);
+  if (!few && !bt->flat_tried) {
+    bt->flat_tried = true;
+    const size_t all = (size_t)(bt->qoff.back() + bt->voff.back()) * sizeof(double);
+    if (all > 0 && hipMalloc((void**)&bt->d_flat, all) != hipSuccess) {
+      (void)hipGetLastError();
+      bt->d_flat = nullptr;
+    }
+  }
+  double* flat = bt->d_flat;
   if (!flat || few) return transfer_by_bucket(bt, hq, hv, oq, ov, to_dev, which);
   const size_t nq = which == 0 ? (size_t)bt->qoff.back() : 0, nv = (size_t)bt->voff.back();
   const gp_batch::Xfer& x = bt->xfer[which];

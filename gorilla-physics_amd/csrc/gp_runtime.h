@@ -141,7 +141,10 @@ struct gp_batch {
   struct Xfer { int at = 0, n = 0; unsigned blocks = 0; };
   gp::XferEntry* d_xfer = nullptr;
   Xfer xfer[4];
-  double* d_flat = nullptr;  // flat staging array of the host transfers, or null
+  // flat staging array (one q, one v) of the host transfers: allocated by the
+  // first one, null where it did not fit
+  double* d_flat = nullptr;
+  bool flat_tried = false;
   void* d_block = nullptr;   // the allocation that holds these and the lanes' offsets
   // The queries' table (gp_dynamics, gp_mass_matrix, gp_dynamics_bias), built
   // on first use: the buckets that the tree kernel takes, the first query_dyn_n
@@ -157,6 +160,7 @@ struct gp_batch {
   size_t terms_cap = 0;
   ~gp_batch() {
     if (d_terms) (void)hipFree(d_terms);
+    if (d_flat) (void)hipFree(d_flat);
     if (d_query) (void)hipFree(d_query);
     if (d_block) (void)hipFree(d_block);
   }

@@ -51,9 +51,10 @@ enum hipStreamCaptureMode { hipStreamCaptureModeThreadLocal };
 #define GP_HOST_UNPOISON(p, n) ((void)0)
 #endif
 constexpr size_t kGpHostGuard = (size_t)1 << 20;
-inline size_t gp_host_malloc_calls = 0;
+inline size_t gp_host_malloc_calls = 0, gp_host_malloc_bytes = 0;
 inline hipError_t hipMalloc(void** p, size_t n) {
   ++gp_host_malloc_calls;
+  gp_host_malloc_bytes += n;
   const size_t body = (n + 15) / 16 * 16;
   char* raw = (char*)std::calloc(body + 2 * kGpHostGuard + 16, 1);
   if (!raw) return hipErrorOutOfMemory;

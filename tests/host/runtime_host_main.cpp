@@ -191,9 +191,39 @@ static void scratch() {
   gp_model_destroy(body);
 }
 
+// A batch whose state only crosses as device arrays has no staging array for
+// host ones; the first host transfer allocates it, once.
+static void staging() {
+  gp_model* m[2] = {lone_body(GP_JOINT_FLOATING), lone_body(GP_JOINT_REVOLUTE)};
+  const int64_t n[2] = {3, 2};
+  gp_batch* b = nullptr;
+  need(gp_batch_create(m, n, 2, nullptr, &b) == GP_OK, "gp_batch_create");
+  const int nq = 3 * 7 + 2, nv = 3 * 6 + 2;
+  std::vector<double> q(nq, 0.5), v(nv, 0.25), q1(nq), v1(nv);
+  size_t at = gp_host_malloc_bytes;
+  auto grown = [&](size_t by, const char* what) {
+    need(gp_host_malloc_bytes - at == by, what);
+    at = gp_host_malloc_bytes;
+  };
+  // host memory is the stand-in's device memory
+  need(gp_batch_set_state_dev(b, q.data(), v.data(), nullptr) == GP_OK, "gp_batch_set_state_dev");
+  need(gp_batch_get_state_dev(b, q1.data(), v1.data(), nullptr) == GP_OK, "gp_batch_get_state_dev");
+  need(q1 == q && v1 == v, "device arrays: the state read back differs");
+  grown(0, "device-array calls allocated memory");
+  need(gp_batch_get_state(b, q1.data(), v1.data()) == GP_OK, "gp_batch_get_state");
+  need(q1 == q && v1 == v, "host arrays: the state read back differs");
+  grown((nq + nv) * sizeof(double), "the first host transfer did not allocate the staging array");
+  need(gp_batch_set_state(b, q1.data(), v1.data()) == GP_OK, "gp_batch_set_state");
+  need(gp_batch_set_tau(b, nullptr) == GP_OK, "gp_batch_set_tau");
+  grown(0, "a later host transfer allocated memory");
+  gp_batch_destroy(b);
+  for (gp_model* x : m) gp_model_destroy(x);
+}
+
 int main(int argc, char** argv) {
   need(argc == 2, "usage: runtime_host <check>");
-  const struct { const char* name; void (*f)(); } checks[] = {{"autotune", autotune}, {"device", device}, {"scratch", scratch}};
+  const struct { const char* name; void (*f)(); } checks[] = {
+      {"autotune", autotune}, {"device", device}, {"scratch", scratch}, {"staging", staging}};
   for (const auto& c : checks)
     if (!std::strcmp(argv[1], c.name)) {
       c.f();

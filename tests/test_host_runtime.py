@@ -34,7 +34,7 @@ def runtime_host(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("check", ["autotune", "device", "scratch"])
+@pytest.mark.parametrize("check", ["autotune", "device", "scratch", "staging"])
 def test_host_side(runtime_host, check):
     p = subprocess.run([runtime_host, check], capture_output=True, text=True, timeout=120)
     assert p.returncode == 0, p.stdout + p.stderr
