@@ -116,9 +116,12 @@ def roofline(work, variant, fp64_kernel, traffic=None, kernel=None):
     """VALU roofline of one measured variant: algorithmic flops of the timed
     steps / the HIP-event time of the timed launches. The peak is the
     mix-weighted one: the shortest time the flops can take is
-    F64 / P64 + F32 / P32 (an FP64 kernel runs both parts at P64)."""
+    F64 / P64 + F32 / P32 (an FP64 kernel runs both parts at P64). An FP64
+    kernel whose formulation needs fewer is credited with those it executes."""
     f32 = float(work["f32_per_batch_step"]) * variant["steps"]
     f64 = float(work["f64_per_batch_step"]) * variant["steps"]
+    if fp64_kernel and "f64_kernel_ops_per_batch_step" in work:
+        f32, f64 = 0.0, float(work["f64_kernel_ops_per_batch_step"]) * variant["steps"]
     if fp64_kernel:
         t_min = (f32 + f64) / (PEAK_TFLOPS["f64"] * 1e12)
     else:
