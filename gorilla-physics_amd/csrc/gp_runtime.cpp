@@ -551,23 +551,26 @@ BucketArgs bucket_args(const Bucket& b, int lanes, const double* tau) {
 }
 
 // Time of one step of one wave of a bucket's compiled kernel in microseconds,
-// by topology and precision (measured on MI355X with 16,384 instances per
-// topology, before the FP64 chains' LDS tier; entries for 5, 7, 9 and 11
-// joints interpolated). Per-lane revolute/prismatic kinds add about a fifth.
+// by topology, precision and whether every joint is revolute (measured on
+// MI355X with as many instances as have a SIMD each: 16,384 of a chain, free
+// body or quadruped, 1,024 trees of 19-26 bodies, whose mean stands for all).
 // Only the ratios matter: they order a grouped launch's buckets and set the
 // serving loop's steps per pool.
 double bucket_step_cost(const Bucket& b, int precision, int lanes_per_tree) {
-  static const double chain_mixed[12] = {0.25, 1.07, 2.13, 3.08, 4.2, 5.27, 6.4, 7.6, 11.5, 15.5, 17.9, 20.2};
-  static const double chain_f64[12] = {0.5, 1.35, 2.77, 4.16, 7.3, 10.5, 14.2, 17.9, 33.4, 48.9, 61.7, 74.5};
+  static const double chain[2][2][12] = {
+      {{0.32, 0.91, 1.98, 3.4, 4.7, 5.9, 8.2, 11.0, 11.5, 14.9, 19.8, 22.1},   // FP64, per-lane joint kinds
+       {0.22, 0.66, 1.51, 2.44, 3.65, 4.6, 5.7, 6.9, 9.7, 11.7, 14.8, 17.2}},  // FP64, all revolute
+      {{0.32, 1.34, 2.31, 3.4, 4.8, 5.8, 7.2, 8.6, 10.4, 11.8, 13.3, 14.7},    // mixed
+       {0.22, 1.0, 2.01, 3.0, 4.1, 5.1, 6.2, 7.3, 8.9, 10.5, 11.9, 13.2}}};
   const bool mixed = precision == GP_PREC_MIXED;
+  const double* of = chain[mixed][b.all_rev];
   const int t = b.fast_topo;
-  if (t >= 1 && t <= 12) return (mixed ? chain_mixed : chain_f64)[t - 1] * (b.all_rev ? 1.0 : 1.2);
-  if (t > TOPO_WELDED && t <= TOPO_WELDED + kMaxWeldedJoints)  // a welded base costs nothing per step
-    return (mixed ? chain_mixed : chain_f64)[t - TOPO_WELDED - 1] * (b.all_rev ? 1.0 : 1.2);
-  if (t == TOPO_QUAD && lanes_per_tree == 1) return mixed ? 29.4 : 116.0;
-  if (t == TOPO_QUAD) return mixed ? 7.0 : 14.3;   // one lane per leg
-  if (t == TOPO_FREE) return mixed ? 1.4 : 1.7;    // four lanes per body, 8 contact points
-  return mixed ? 20.0 : 75.0;
+  if (t >= 1 && t <= 12) return of[t - 1];
+  if (t > TOPO_WELDED && t <= TOPO_WELDED + kMaxWeldedJoints) return of[t - TOPO_WELDED - 1];  // the base costs nothing
+  if (t == TOPO_QUAD && lanes_per_tree == 1) return mixed ? 37.4 : 120.0;
+  if (t == TOPO_QUAD) return mixed ? 6.6 : 21.8;  // one lane per leg
+  if (t == TOPO_FREE) return mixed ? 1.3 : 1.4;   // four lanes per body, 8 contact points, four touching
+  return mixed ? 11.0 : 14.0;
 }
 
 }  // namespace gp
@@ -1381,14 +1384,14 @@ int gp_batch_get_vdot(gp_batch* bt, double* vdot) {
 // estimate of both in us. A wave of the tree kernel goes through its levels
 // one after the other and loads a line per body and field, which instances of
 // many bodies share less, 2,048 waves at a time; the plain kernel's time is its
-// bodies' chain of dependent scratch accesses, then their bytes. So long chains in large batches are the plain
-// kernel's. Tree / plain kernel, us, at 4,096, 16,384 and 65,536 instances:
-// chains of 12 bodies 31 / 136, 82 / 150, 208 / 285; of 16 41 / 185, 114 / 205,
-// 367 / 402; of 22 80 / 252, 230 / 291, 838 / 521; of 32 167 / 376, 364 / 501,
-// 1,299 / 762; of 40 221 / 470, 760 / 645, 2,852 / 940; of 64 432 / 702, 1,306 /
-// 1,033, 4,965 / 1,500; trees of 64 bodies in 4 levels 105 / 730, 307 / 990, 1,410
-// / 1,420. Of 160 sizes tried the estimate takes the slower one at one, by 4 %
-// (32,768 chains of 24).
+// bodies' chain of dependent scratch accesses, then their bytes. So long chains
+// in large batches are the plain kernel's. Tree / plain kernel, us, at 4,096,
+// 16,384 and 65,536 instances: chains of 12 bodies 31 / 136, 82 / 150, 208 / 285;
+// of 16 41 / 185, 114 / 205, 367 / 402; of 22 80 / 252, 230 / 291, 838 / 521; of
+// 32 167 / 376, 364 / 501, 1,299 / 762; of 40 221 / 470, 760 / 645, 2,852 / 940;
+// of 64 432 / 702, 1,306 / 1,033, 4,965 / 1,500; trees of 64 bodies in 4 levels
+// 105 / 730, 307 / 990, 1,410 / 1,420. Of 160 sizes tried the estimate takes the
+// slower one at one, by 4 % (32,768 chains of 24).
 static bool tree_dynamics_faster(const Bucket& b) {
   const double waves = (double)fast_threads(TOPO_TREE, b.B, b.nb) / 64.0, bodies = 64 / b.nb * b.nb;
   const double tree = waves / 2048.0 * (bodies * (0.1 + b.nb / 130.0) + 2.0 * (b.max_depth + 1));
