@@ -204,8 +204,8 @@ int launch_fast_step(int topo_id, int precision, const BucketArgs& a, double dt,
 int launch_fast_rk_step(int topo_id, int precision, int integrator, const BucketArgs& a, double dt, int n_steps,
                         int block, void* stream);
 size_t plain_scratch_doubles(int nb, int nq, int nv, int Bp);
-// velocity stepping (ccd = 1: with continuous collision detection), FP64, one
-// step per launch; scratch as vs_layout
+// velocity stepping (ccd = 1: with continuous collision detection), FP64,
+// n_steps steps per launch; scratch as vs_layout
 int launch_vs_step(const BucketArgs& a, double dt, int ccd, int n_steps, void* stream);
 // the same step with one instance per wave, the same bits; vs_wave_ok: whether
 // the bucket's sizes fit and its instances are few enough for it to be faster

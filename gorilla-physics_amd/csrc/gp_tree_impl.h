@@ -84,7 +84,7 @@ inline bool tree_topology_ok(int nb, const int* parent) {
   return true;
 }
 
-// L^T D L of a floating joint's 6x6 inertia, packed by rows: unit lower factor
+// L D L^T of a floating joint's 6x6 inertia, packed by rows: unit lower factor
 // below the diagonal, reciprocal pivots on it; false if a pivot is not positive.
 __device__ __forceinline__ bool ldl6(const ai6<double>& I, double (&L)[21]) {
   L[0] = I.A.xx;

@@ -1,8 +1,9 @@
 // gp_vstep.hip — velocity stepping with and without continuous collision
-// detection (integrators.rs:42-175, dynamics.rs:366-742): one instance per
-// lane, FP64, runtime topology, one step per launch.
+// detection (integrators.rs:42-175, dynamics.rs:366-742), FP64, runtime
+// topology, n_steps steps per launch: one instance per lane (vs_step_kernel)
+// or per wave (vs_wave_kernel, below), the same bits.
 //
-// Per lane and step:
+// Per instance and step:
 //  1. free velocity v_free = v + dt M^-1 (tau + springs - c(q, v)) by the
 //     articulated-body algorithm without contact forces (dynamics.rs:375-395);
 //  2. contacts: contact points inside a half-space and sphere colliders
@@ -21,8 +22,9 @@
 // reach a half-space with v_next, and the rest of the step is stepped again;
 // a sphere that ended a cut touches that half-space in the next round.
 //
-// Every per-lane array is a [k][Bp] column block of the bucket's scratch
-// (vs_layout), so each access of a wavefront is one coalesced 512-byte line.
+// One instance per lane: every per-lane array is a [k][Bp] column block of the
+// bucket's scratch (vs_layout), so each access of a wavefront is one coalesced
+// 512-byte line. One instance per wave: the arrays are in LDS (vw_layout).
 #include "gp_cone.h"
 #include "gp_plain_impl.h"
 
@@ -1123,8 +1125,12 @@ int launch_vs_step(const BucketArgs& a, double dt, int ccd, int n_steps, void* s
 // The wave's lanes hold the program's rows, the bodies and the coordinates, and
 // a workgroup's LDS its working set. The line lies where the instances no longer
 // have a SIMD each: until then a launch takes one instance's time, which is the
-// shorter one at any number of contacts, and from there it doubles, where the
-// lane kernel's stays. Two steps, lane / wave, ms, at 64, 1,024 and 2,048 instances:
+// shorter one at any number of contacts; past it the wave kernel's time doubles
+// and that of instances in flight is longer than the lane kernel's. Whether
+// instances touch is not known when the launch is made, and none may be slower
+// than on the lane kernel alone. Instances that do touch pay for it: they
+// would be faster on the wave kernel up to several thousand (the crossing lies
+// between 2,048 and 16,384 standing quadrupeds). Two steps, lane / wave, ms, at 64, 1,024 and 2,048 instances:
 // quadrupeds on four feet 8.3 / 1.09, 8.8 / 1.25, 9.0 / 2.2 (and 11.8 / 14.8 at
 // 16,384), in flight 0.200 / 0.131, 0.206 / 0.147, 0.207 / 0.297; 8-joint arms
 // with one contact 1.04 / 0.38, 1.21 / 0.44, 1.22 / 0.83, with none 0.155 / 0.098,

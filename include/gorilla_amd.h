@@ -187,7 +187,8 @@ typedef struct gp_batch_opts {
                                 one instance's contact points, 1/2/4/8 (0 = 4);
                                 velocity stepping of a lone floating body with
                                 at most 8 contact candidates: 1 = one lane
-                                per body, else 8 lanes per body             */
+                                per body, else 4 lanes per body (8 once more
+                                than four of its candidates touch)          */
   int32_t use_graph;         /* capture multi-launch rollouts in a hipGraph   */
                              /* (a chunk of one kernel is launched directly)  */
   int32_t separate_launches; /* 1: one launch per topology bucket instead of
